@@ -374,21 +374,61 @@ bool config_built(const fl::FwdArgs& a, int cfg) {
   return a.head_dim == 64 && cfg != fl::kCfgW1 && cfg != fl::kCfgW2;
 }
 
+// Head dim 128 (fp16 and bf16 alike; a sweep of 1-128 heads by N 512-8192
+// in bf16, both masks, us per call).  The key-range splits double or
+// quadruple the waves of a problem and halve its longest walk, so they win
+// while they fit one round of the CUs; the groups without a split read each
+// tile for more rows, which counts once the chip is full:
+//  - at most one 64-row group per CU, causal 1.5 (their lengths differ):
+//    the split on 64-row groups (B2 H8 N1024 14.3 against 17.4 for the 4-wave
+//    groups, B1 H4 N4096 causal 32.9 against 51.6, B2 H8 N1536 causal 20.5
+//    against 24.0; with 512 groups B2 H8 N2048 42.0 against 35.9);
+//  - square causal from 1024 keys with at most one pair of 64-row blocks per
+//    CU: the pairs (B2 H8 N2048 26.5 against 31.0 and 29.4 for the 128-row
+//    split, B1 H4 N8192 76.8 against 101.6 and 89.6; below 1024 keys a pair's
+//    second start-up costs more, B4 H16 N512 15.3 against 13.8);
+//  - from 1536 keys, at most one 128-row group per CU, causal 1.5: the split
+//    on 128-row groups (B2 H8 N1536 24.0 against 24.9, B1 H4 N8192 118
+//    against 127, B2 H8 N3000 causal 43.3 against 49.4; at 1024 keys B2 H16
+//    22.0 against 21.6);
+//  - square causal from 4096 keys with at most one pair of 128-row blocks per
+//    CU: the pairs (B2 H8 N4096 68.4 against 72.1 and 70.1);
+//  - 256-row groups, non-causal: when one round of them holds what 128-row
+//    groups need a second for (B2 H8 N3000 73.6 against 76.0, B2 H16 N2048
+//    61.2 against 63.9, B2 H16 N3000, two rounds, 149 against 133), and from
+//    4096 keys (B2 H8 N8192 431 against 454); causal from 4096 keys with two
+//    rounds of them (B1 H16 N16384 894 against 923, B2 H8 N8192 231 against
+//    237);
+//  - else 128-row groups of 4 waves, two per CU.
+int select_d128(const fl::FwdArgs& a) {
+  const int64_t cus = fl::device_cus();
+  auto wgs = [&](int64_t br) { return (a.seq + br - 1) / br * (int64_t)a.batch_heads; };
+  const bool square = a.causal && a.seq == a.seq_k;
+  const int64_t pairs64 = (((int64_t)a.seq + 63) / 64 + 1) / 2 * a.batch_heads;
+  const int64_t most = a.causal ? cus + cus / 2 : cus;
+  if (wgs(64) <= most) return fl::kCfgSplit2W2;
+  if (square && a.seq_k >= 1024 && pairs64 <= cus) return fl::kCfgPairW2;
+  if (a.seq_k >= 1536 && wgs(128) <= most) return fl::kCfgSplit2;
+  if (square && a.seq_k >= 4096 && wgs(128) <= 2 * cus) return fl::kCfgPair;
+  if (!a.causal && wgs(128) > cus && wgs(256) <= cus) return fl::kSlotW8Config;
+  if (a.seq_k >= 4096 && wgs(256) >= (a.causal ? 2 : 1) * cus) return fl::kSlotW8Config;
+  return fl::kSlotW4Config;
+}
+
 // bf16 at head_dim 64 follows the fp16 dispatcher where it picks the
 // streaming kernel, the key quarters, a key-range split or block pairs, and
 // the 4-wave groups for at most 32 query rows over at least as many heads
 // as CUs (bf16 one pass: 0-5% faster than the 256-row groups, B8 H32 N_q 1
-// N_k 8192 92.1 against 96.9 us); otherwise (and at head_dim 128) one of the
-// slot-scheduled groups by the rule below.
+// N_k 8192 92.1 against 96.9 us); otherwise one of the slot-scheduled groups
+// by the rule below.
 int select_any(const fl::FwdArgs& a) {
   if (!narrow_configs(a)) return select_fa2(a);
-  if (a.head_dim == 64) {
-    const int c = select_fa2(a);
-    if (c == fl::kCfgSplit2 || c == fl::kCfgSplit2W2 || c == fl::kCfgPair || c == fl::kCfgPairW2 ||
-        c == fl::kStreamConfig || c == fl::kQuarterConfig)
-      return c;
-    if (a.seq <= 32 && a.batch_heads >= fl::device_cus()) return fl::kSlotW4Config;
-  }
+  if (a.head_dim == 128) return select_d128(a);
+  const int c = select_fa2(a);
+  if (c == fl::kCfgSplit2 || c == fl::kCfgSplit2W2 || c == fl::kCfgPair || c == fl::kCfgPairW2 ||
+      c == fl::kStreamConfig || c == fl::kQuarterConfig)
+    return c;
+  if (a.seq <= 32 && a.batch_heads >= fl::device_cus()) return fl::kSlotW4Config;
   const int64_t cus = fl::device_cus();
   const int64_t wgs256 = (a.seq + 255) / 256 * (int64_t)a.batch_heads;
   return (!a.causal && a.seq_k >= 4096 && wgs256 >= cus) ? fl::kSlotW8Config

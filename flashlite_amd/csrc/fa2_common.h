@@ -362,6 +362,16 @@ __device__ __forceinline__ void fetch_tile_z(const i32x4_t& rs, const uint8_t* s
   }
 }
 
+// Segment `i` of this wave's share of such a fetch alone: `tb` is the tile's
+// byte offset, min(t, tzero) * f.tile_bytes.
+template <int kSegs>
+__device__ __forceinline__ void fetch_seg(const i32x4_t& rs, const uint8_t* slot, int tb, int i,
+                                          int wave, const FetchOff<kSegs>& f) {
+  const int voff = tb + f.lane[i];
+  const uint32_t lds_base = (uint32_t)(uintptr_t)(slot + 1024 * (wave * kSegs + i));
+  asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" : : "v"(voff), "s"(rs), "{m0}"(lds_base));
+}
+
 // DMA of the 32 query rows [q, q + 32) of a head (rows >= N_q read as
 // zeros) into `qblk`, laid out as the first half of a K tile (Rows::
 // set_q_lds reads it): 4 fetches of 1 KiB, counted by vmcnt, or with kParts

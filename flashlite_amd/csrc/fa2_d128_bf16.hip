@@ -1,0 +1,11 @@
+// Head dim 128, bf16: see fa2_d128_kernel.h.
+
+#include "fa2_d128_kernel.h"
+
+namespace fl {
+
+hipError_t launch_d128_bf16(const FwdArgs& a, int cfg, hipStream_t stream) {
+  return launch_d128_t<__bf16>(a, cfg, stream);
+}
+
+}  // namespace fl

@@ -27,11 +27,9 @@ bool stream_config_fits(const FwdArgs& a) {
 }
 
 hipError_t launch_fa2(const FwdArgs& a, int cfg, hipStream_t stream) {
-  if (a.head_dim == 128) {
-    if (cfg == kSlotW8Config) return launch_d128(a, 8, stream);
-    if (cfg == kSlotW4Config) return launch_d128(a, 4, stream);
-    return hipErrorInvalidValue;
-  }
+  if (a.head_dim == 128)
+    return a.dtype == kDtypeBF16 ? launch_d128_bf16(a, cfg, stream)
+                                 : launch_d128_f16(a, cfg, stream);
   if (a.dtype == kDtypeBF16) {
     if (cfg == kSlotW8Config) return launch_slot(a, 8, stream);
     if (cfg == kSlotW4Config) return launch_slot(a, 4, stream);

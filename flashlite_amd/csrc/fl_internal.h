@@ -65,8 +65,9 @@ extern const Fa2Config kFa2Configs[kNumFa2Configs];
 
 // Launches the FA2 kernel for configuration `cfg` on `stream`.  fp16 at
 // head_dim 64 has every configuration; bf16 at head_dim 64 all but the
-// pipelined ones (kCfgW1, kCfgW2); head_dim 128 the slot-scheduled ones
-// (kSlotW8Config, kSlotW4Config).
+// pipelined ones (kCfgW1, kCfgW2); head_dim 128 the slot-scheduled ones and
+// their key-range splits and block pairs (kSlotW8Config, kSlotW4Config,
+// kCfgSplit2, kCfgSplit2W2, kCfgPair, kCfgPairW2).
 hipError_t launch_fa2(const FwdArgs& a, int cfg, hipStream_t stream);
 constexpr int kStreamMaxKeys = 256;
 constexpr int kStreamMaxRowStride = 1 << 22;
@@ -121,7 +122,8 @@ hipError_t launch_slot_split(const FwdArgs& a, int waves, hipStream_t stream);  
 hipError_t launch_slot_pair(const FwdArgs& a, int waves, hipStream_t stream);   // fa2_slot.hip
 hipError_t launch_stream(const FwdArgs& a, hipStream_t stream);            // fa2_stream.hip
 hipError_t launch_quarter(const FwdArgs& a, hipStream_t stream);           // fa2_short.hip
-hipError_t launch_d128(const FwdArgs& a, int waves, hipStream_t stream);   // fa2_d128.hip
+hipError_t launch_d128_f16(const FwdArgs& a, int cfg, hipStream_t stream);   // fa2_d128.hip
+hipError_t launch_d128_bf16(const FwdArgs& a, int cfg, hipStream_t stream);  // fa2_d128_bf16.hip
 
 // Split-KV ("flash-decoding"): `waves` (1, 2 or 4) waves of 32 query rows
 // per work-group, the key range cut into `nsplit` chunks whose partial
