@@ -91,6 +91,14 @@ fa2_fwd_slot_kernel(const T* Q, const T* __restrict__ K, const T* __restrict__ V
   constexpr int kSegs = 8 / W;
   constexpr int kDmaPerIter = 2 * kSegs;
   constexpr int kAhead = 6;  // slots between an operand's LDS read and its MFMA
+  // A DMA instruction waits at issue while the CU's memory pipeline is busy:
+  // the iteration's fetches go out one every kDmaEvery slots instead of all
+  // at its start (64-row groups, 8 per wave: B2 H8 N1024 9.6 -> 9.15 us, B1 H4
+  // N2048 13.6 -> 12.5, pairs B1 H2 N16384 causal 93.0 -> 87.4; the 8-wave
+  // groups and the 128-row split and pairs 0-2%).  Not in the 4-wave groups,
+  // two per CU, where the causal ones lost 2% at B2 H8 N4096 and N2048.
+  constexpr bool kSpread = W != 4 || SPLIT == 2;
+  constexpr int kDmaEvery = 16 / kDmaPerIter;
   // LDS reads of the first kAhead slots (K slots: 1, V slots: 2).
   constexpr int kTailReads = kAhead + kAhead / 2;
   constexpr int kRingBytes = kSlots * kTileBytes;
@@ -270,8 +278,16 @@ fa2_fwd_slot_kernel(const T* Q, const T* __restrict__ K, const T* __restrict__ V
     constexpr bool kMasked = decltype(masked)::value;
     constexpr int Kd = decltype(kind)::value;
     constexpr bool kFold = (Kd & kLast) != 0;
-    fetch_tile_z<kSegs>(rk, rings.kslot(Ic<I + FK>{}), tbeg + j + FK, tzero, rw, fk);
-    fetch_tile_z<kSegs>(rv, rings.vslot(Ic<I + FV>{}), tbeg + j + FV, tzero, rw, fv);
+    const int tbk = min(tbeg + j + FK, tzero) * fk.tile_bytes;
+    const int tbv = min(tbeg + j + FV, tzero) * fv.tile_bytes;
+    auto fetch = [&](auto n) __attribute__((always_inline)) {  // K segments, then V's
+      constexpr int d = decltype(n)::value;
+      if constexpr (d < kSegs)
+        fetch_seg<kSegs>(rk, rings.kslot(Ic<I + FK>{}), tbk, d, rw, fk);
+      else
+        fetch_seg<kSegs>(rv, rings.vslot(Ic<I + FV>{}), tbv, d - kSegs, rw, fv);
+    };
+    if constexpr (!kSpread) static_for(std::make_integer_sequence<int, kDmaPerIter>{}, fetch);
     V8 op[16];
     V8 top[kLastTail];  // kLast: the tail MFMAs' operands
 #pragma unroll
@@ -291,6 +307,7 @@ fa2_fwd_slot_kernel(const T* Q, const T* __restrict__ K, const T* __restrict__ V
           rows.template mfma_slot<L, true>(op[L], S, Pp);
       }
       if constexpr (kFence) __builtin_amdgcn_sched_barrier(0);
+      if constexpr (kSpread && L % kDmaEvery == 0) fetch(Ic<L / kDmaEvery>{});
       if constexpr (L + kAhead < 16) {
         constexpr int La = L + kAhead;
         if constexpr (runs(Kd, La)) {
