@@ -105,6 +105,10 @@ int check_pointers(const fl_attn_params* p, fl::FwdArgs* a, const char* who, uin
   return FL_OK;
 }
 
+// The public table's rule: what fl_attn_select_config reports, and the base
+// of select_d64, which launches by newer measurements where they differ (its
+// answers for given shapes are part of the interface; callers look them up).
+//
 // Tile-configuration choice for the device's CUs (fl::device_cus(): 256 on
 // an MI355X seen whole, where the rules below were measured; every
 // configuration computes the same result).  Key ranges of at most 256 keys
@@ -379,6 +383,8 @@ bool config_built(const fl::FwdArgs& a, int cfg) {
 // quadruple the waves of a problem and halve its longest walk, so they win
 // while they fit one round of the CUs; the groups without a split read each
 // tile for more rows, which counts once the chip is full:
+//  - at most one 32-row block per CU: the 32-row groups (fa2_rows32.hip; with
+//    384 blocks B2 H12 N512 9.8 against 8.9 for the 64-row split);
 //  - at most one 64-row group per CU, causal 1.5 (their lengths differ):
 //    the split on 64-row groups (B2 H8 N1024 14.3 against 17.4 for the 4-wave
 //    groups, B1 H4 N4096 causal 32.9 against 51.6, B2 H8 N1536 causal 20.5
@@ -406,6 +412,7 @@ int select_d128(const fl::FwdArgs& a) {
   const bool square = a.causal && a.seq == a.seq_k;
   const int64_t pairs64 = (((int64_t)a.seq + 63) / 64 + 1) / 2 * a.batch_heads;
   const int64_t most = a.causal ? cus + cus / 2 : cus;
+  if (wgs(32) <= cus && !(a.seq <= 32 && a.batch_heads >= cus)) return fl::kRows32Config;
   if (wgs(64) <= most) return fl::kCfgSplit2W2;
   if (square && a.seq_k >= 1024 && pairs64 <= cus) return fl::kCfgPairW2;
   if (a.seq_k >= 1536 && wgs(128) <= most) return fl::kCfgSplit2;
@@ -415,24 +422,77 @@ int select_d128(const fl::FwdArgs& a) {
   return fl::kSlotW4Config;
 }
 
-// bf16 at head_dim 64 follows the fp16 dispatcher where it picks the
+// Head dim 64, fp16 and bf16 (sweeps of 1-1024 heads by N 40-8192, both
+// masks, us per call; fp16 figures, bf16 within 3% of them):
+//  - at most one 32-row block per CU, square causal 1.5 (their lengths
+//    differ; 1.25-1.5 non-causal lose 3-11%): the 32-row groups (figures in
+//    fa2_rows32.hip; B2 H8 N640 causal 7.35 against 7.9), but for 257-512 keys
+//    with at most 5/8 of a block per CU the key quarters, whose waves hold
+//    both their tiles at once (B1 H8 N384 5.05 against 5.35, B1 H16 N300 5.28
+//    against 5.56; at 256 blocks B2 H8 N512 7.3 against 5.6).  Q rows must lie
+//    within the buffer offsets of a block (2^24 elements apart);
+//  - up to 256 keys beyond that: the 64-row split while it fits one round and
+//    has four tiles (B4 H16 N256 5.95 against 6.3; at N192 5.9 against 5.7),
+//    the streaming groups from 1024 units of 256 rows and 128 keys (B32 H32
+//    N128 16.1 against 16.9, causal N256 32.7 against 39.2) or 512 causal ones
+//    past 192 keys (B16 H32 N256 17.4 against 19.4), else the 4-wave groups
+//    (B8 H16 N256 7.7 against 9.0 streaming, B16 H32 N96 8.6 against 10.0);
+//  - at most one 64-row group per CU, causal from 1280 keys 1.5: the 64-row
+//    split (B2 H16 N512 7.1 against 11.3 on the key quarters' 8-wave groups,
+//    B2 H8 N1280 causal 12.1 against 14.2, B1 H8 N3000 causal 20.1 against
+//    22.0; at N640-768 causal with 1.25-1.5 it lost 10-15%);
+//  - square causal from 1792 keys with at most one pair of 64-row blocks per
+//    CU: the 64-row pairs (B2 H8 N1999 17.9 against 18.4 for the 128-row split;
+//    N1024 over 32 heads 14.3 against 13.4);
+//  - non-causal from 1280 keys with at most one 128-row group per CU: the
+//    128-row split (B2 H8 N1280 12.9 against 14.0; B2 H16 N1024 14.25 against
+//    14.1);
+//  - fp16, non-causal from 2048 keys with more 256-row groups than CUs: those
+//    only from 4096 keys or where their last round is nearly full (B2 H16
+//    N3000, 1.5 rounds, 91.3 against 79.9 on the 4-wave groups).
+// Beyond these, fp16 follows the public rule; bf16 does where that picks the
 // streaming kernel, the key quarters, a key-range split or block pairs, and
-// the 4-wave groups for at most 32 query rows over at least as many heads
-// as CUs (bf16 one pass: 0-5% faster than the 256-row groups, B8 H32 N_q 1
-// N_k 8192 92.1 against 96.9 us); otherwise one of the slot-scheduled groups
-// by the rule below.
-int select_any(const fl::FwdArgs& a) {
-  if (!narrow_configs(a)) return select_fa2(a);
-  if (a.head_dim == 128) return select_d128(a);
+// otherwise takes a slot-scheduled group (4 waves for at most 32 query rows
+// over as many heads as CUs: 0-5% faster than 8).
+int select_d64(const fl::FwdArgs& a) {
+  const int64_t cus = fl::device_cus();
+  auto wgs = [&](int64_t br) { return (a.seq + br - 1) / br * (int64_t)a.batch_heads; };
+  const bool square = a.causal && a.seq == a.seq_k;
+  const bool few = a.seq <= 32 && a.batch_heads >= cus;  // decode over many heads
+  if (!few && a.q_sr <= (1 << 24) && wgs(32) <= (square ? cus + cus / 2 : cus)) {
+    if (a.seq_k > 256 && fl::quarter_config_fits(a) && 8 * wgs(32) <= 5 * cus)
+      return fl::kQuarterConfig;
+    return fl::kRows32Config;
+  }
+  if (a.seq_k <= 256) {
+    if (a.seq_k > 192 && wgs(64) <= cus) return fl::kCfgSplit2W2;
+    if (fl::stream_config_fits(a) &&
+        ((a.seq_k >= 128 && wgs(256) >= 4 * cus) ||
+         (a.causal && a.seq_k > 192 && wgs(256) >= 2 * cus)))
+      return fl::kStreamConfig;
+    return fl::kSlotW4Config;
+  }
+  if (few) return fl::kSlotW4Config;
+  if (wgs(64) <= (a.causal && a.seq_k >= 1280 ? cus + cus / 2 : cus)) return fl::kCfgSplit2W2;
+  const int64_t pairs64 = (((int64_t)a.seq + 63) / 64 + 1) / 2 * a.batch_heads;
+  if (square && a.seq_k >= 1792 && pairs64 <= cus) return fl::kCfgPairW2;
+  if (!a.causal && a.seq_k >= 1280 && wgs(128) <= cus) return fl::kCfgSplit2;
   const int c = select_fa2(a);
+  if (a.dtype == fl::kDtypeF16) {
+    const int64_t g = wgs(256), rounds = (g + cus - 1) / cus;
+    if (c == fl::kSlotW8Config && a.seq_k < 4096 && rounds > 1 && 10 * g < 9 * rounds * cus)
+      return fl::kSlotW4Config;
+    return c;
+  }
   if (c == fl::kCfgSplit2 || c == fl::kCfgSplit2W2 || c == fl::kCfgPair || c == fl::kCfgPairW2 ||
       c == fl::kStreamConfig || c == fl::kQuarterConfig)
     return c;
-  if (a.seq <= 32 && a.batch_heads >= fl::device_cus()) return fl::kSlotW4Config;
-  const int64_t cus = fl::device_cus();
-  const int64_t wgs256 = (a.seq + 255) / 256 * (int64_t)a.batch_heads;
-  return (!a.causal && a.seq_k >= 4096 && wgs256 >= cus) ? fl::kSlotW8Config
-                                                           : fl::kSlotW4Config;
+  return (!a.causal && a.seq_k >= 4096 && wgs(256) >= cus) ? fl::kSlotW8Config
+                                                            : fl::kSlotW4Config;
+}
+
+int select_any(const fl::FwdArgs& a) {
+  return a.head_dim == 128 ? select_d128(a) : select_d64(a);
 }
 
 int fwd_ex(const fl_attn_params_ex* p, int32_t config, void* stream, int dtype, const char* who) {
@@ -543,7 +603,7 @@ int fl_attn_fwd_f16_cfg(const fl_attn_params* p, int32_t config, void* stream) {
   if (empty_problem(a)) return FL_OK;
   rc = check_pointers(p, &a, "fl_attn_fwd_f16", 16);
   if (rc != FL_OK) return rc;
-  const int cfg = config < 0 ? select_fa2(a) : config;
+  const int cfg = config < 0 ? select_any(a) : config;
   const hipError_t e = fl::launch_fa2(a, cfg, static_cast<hipStream_t>(stream));
   if (e != hipSuccess)
     return fail(FL_ERR_LAUNCH, "fl_attn_fwd_f16: launch failed: %s", hipGetErrorString(e));
@@ -588,7 +648,7 @@ int fl_attn_fwd_f16_splitkv(const fl_attn_params_ex* p, int32_t num_splits, void
   const KvPlan plan = plan_kvsplit(a, num_splits);
   hipError_t e;
   if (plan.nsplit == 0) {  // the library's choice: one pass, no workspace
-    e = fl::launch_fa2(a, select_fa2(a), static_cast<hipStream_t>(stream));
+    e = fl::launch_fa2(a, select_any(a), static_cast<hipStream_t>(stream));
   } else {
     if (workspace == nullptr || workspace_bytes < plan.bytes)
       return fail(FL_ERR_INVALID_ARGUMENT, "%s: workspace of %lld bytes needed (got %lld%s)", who,
@@ -617,7 +677,7 @@ int fl_attn_fwd_f16_splitkv_noalloc(const fl_attn_params_ex* p, int32_t num_spli
                 (long long)plan.bytes, (long long)FL_ATTN_SCRATCH_BYTES);
   hipError_t e;
   if (plan.nsplit == 0) {
-    e = fl::launch_fa2(a, select_fa2(a), static_cast<hipStream_t>(stream));
+    e = fl::launch_fa2(a, select_any(a), static_cast<hipStream_t>(stream));
   } else {
     void* s = nullptr;
     rc = scratch_for_current_device(&s, who);

@@ -1,6 +1,6 @@
 // Tile configurations of the FA2 forward and their dispatch to the
 // schedule that implements each (fa2_pipe.hip, fa2_slot.hip, fa2_stream.hip,
-// fa2_short.hip, fa2_d128.hip).  The dispatcher that picks a configuration for a problem is
+// fa2_short.hip, fa2_d128.hip, fa2_rows32.hip).  The dispatcher that picks a configuration for a problem is
 // capi.hip's select_fa2.
 
 #include "fl_internal.h"
@@ -27,6 +27,7 @@ bool stream_config_fits(const FwdArgs& a) {
 }
 
 hipError_t launch_fa2(const FwdArgs& a, int cfg, hipStream_t stream) {
+  if (cfg == kRows32Config) return launch_rows32(a, stream);
   if (a.head_dim == 128)
     return a.dtype == kDtypeBF16 ? launch_d128_bf16(a, cfg, stream)
                                  : launch_d128_f16(a, cfg, stream);

@@ -61,13 +61,16 @@ constexpr int kCfgPair = 8;         // br128_bc64_w4x2_pair
 // The same with two 64-row blocks per work-group, 2 x 2 waves.
 constexpr int kCfgPairW2 = 9;       // br64_bc64_w2x2_pair
 constexpr int kNumFa2Configs = 10;
+// Internal, outside the public table: groups of 32 query rows, the key tiles
+// dealt to 4 or 8 waves (fa2_rows32.hip), any element type and head dim.
+constexpr int kRows32Config = kNumFa2Configs;
 extern const Fa2Config kFa2Configs[kNumFa2Configs];
 
 // Launches the FA2 kernel for configuration `cfg` on `stream`.  fp16 at
 // head_dim 64 has every configuration; bf16 at head_dim 64 all but the
 // pipelined ones (kCfgW1, kCfgW2); head_dim 128 the slot-scheduled ones and
 // their key-range splits and block pairs (kSlotW8Config, kSlotW4Config,
-// kCfgSplit2, kCfgSplit2W2, kCfgPair, kCfgPairW2).
+// kCfgSplit2, kCfgSplit2W2, kCfgPair, kCfgPairW2); every type kRows32Config.
 hipError_t launch_fa2(const FwdArgs& a, int cfg, hipStream_t stream);
 constexpr int kStreamMaxKeys = 256;
 constexpr int kStreamMaxRowStride = 1 << 22;
@@ -122,6 +125,7 @@ hipError_t launch_slot_split(const FwdArgs& a, int waves, hipStream_t stream);  
 hipError_t launch_slot_pair(const FwdArgs& a, int waves, hipStream_t stream);   // fa2_slot.hip
 hipError_t launch_stream(const FwdArgs& a, hipStream_t stream);            // fa2_stream.hip
 hipError_t launch_quarter(const FwdArgs& a, hipStream_t stream);           // fa2_short.hip
+hipError_t launch_rows32(const FwdArgs& a, hipStream_t stream);            // fa2_rows32.hip
 hipError_t launch_d128_f16(const FwdArgs& a, int cfg, hipStream_t stream);   // fa2_d128.hip
 hipError_t launch_d128_bf16(const FwdArgs& a, int cfg, hipStream_t stream);  // fa2_d128_bf16.hip
 

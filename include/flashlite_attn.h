@@ -208,8 +208,10 @@ const char* fl_attn_config_name(int32_t config);
  * versions of the library; names do not, so a caller that forces a
  * configuration should look its id up by name. */
 int fl_attn_config_id(const char* name);
-/* Returns the configuration fl_attn_fwd_f16 would launch for `p`, or -1 if
- * `p` is rejected (the reason is in fl_attn_last_error()). */
+/* Returns the public table's choice for `p`, or -1 if `p` is rejected (the
+ * reason is in fl_attn_last_error()).  fl_attn_fwd_f16 launches it unless a
+ * newer measurement favours another one for the shape, which may be internal
+ * to the library (32-row groups, for problems of few query rows). */
 int fl_attn_select_config(const fl_attn_params* p);
 
 #ifdef __cplusplus
