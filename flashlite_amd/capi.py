@@ -36,6 +36,8 @@ EXPORTED = (
     "fl_attn_fwd_f16_splitkv_noalloc",
     "fl_attn_splitkv_noalloc_bytes",
     "fl_attn_config_id",
+    "fl_attn_workspace_bytes",
+    "fl_attn_fwd_ws",
 )
 
 SCRATCH_BYTES = 8 << 20  # FL_ATTN_SCRATCH_BYTES
@@ -110,6 +112,11 @@ def load(path: str = LIB_PATH) -> ctypes.CDLL:
     lib.fl_attn_fwd_bf16_ex.argtypes = [ctypes.POINTER(FlAttnParamsEx), ctypes.c_int32,
                                         ctypes.c_void_p]
     lib.fl_attn_fwd_bf16_ex.restype = ctypes.c_int
+    lib.fl_attn_workspace_bytes.argtypes = [ctypes.POINTER(FlAttnParamsEx), ctypes.c_int32]
+    lib.fl_attn_workspace_bytes.restype = ctypes.c_int64
+    lib.fl_attn_fwd_ws.argtypes = [ctypes.POINTER(FlAttnParamsEx), ctypes.c_int32, ctypes.c_void_p,
+                                   ctypes.c_int64, ctypes.c_void_p]
+    lib.fl_attn_fwd_ws.restype = ctypes.c_int
     lib.fl_attn_splitkv_workspace_bytes.argtypes = [ctypes.POINTER(FlAttnParamsEx), ctypes.c_int32]
     lib.fl_attn_splitkv_workspace_bytes.restype = ctypes.c_int64
     lib.fl_attn_fwd_f16_splitkv.argtypes = [ctypes.POINTER(FlAttnParamsEx), ctypes.c_int32,
@@ -197,6 +204,21 @@ def tensor_params_ex(q, k, v, o, sm_scale=0.0, causal=False, lse=None) -> FlAttn
     base = tensor_params(q, k, v, o, sm_scale, causal)
     strides = [tuple(int(s) for s in t.stride()[:3]) for t in (q, k, v, o)]
     return make_params_ex(base, *strides, lse=0 if lse is None else lse.data_ptr())
+
+
+DTYPE_F16 = 0  # FL_DTYPE_F16
+DTYPE_BF16 = 1
+
+
+def workspace_bytes(params: FlAttnParamsEx, dtype: int) -> int:
+    """``fl_attn_workspace_bytes``: 0 for one pass, -1 if `params` is rejected."""
+    return int(load().fl_attn_workspace_bytes(ctypes.byref(params), dtype))
+
+
+def fwd_ws(params: FlAttnParamsEx, dtype: int, workspace: int, nbytes: int, stream: int = 0) -> int:
+    """``fl_attn_fwd_ws``; returns the status code."""
+    return load().fl_attn_fwd_ws(ctypes.byref(params), dtype, workspace or None, nbytes,
+                                 stream or None)
 
 
 def naive(params: FlAttnParams, stream: int = 0) -> int:

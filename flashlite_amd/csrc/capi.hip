@@ -105,9 +105,9 @@ int check_pointers(const fl_attn_params* p, fl::FwdArgs* a, const char* who, uin
   return FL_OK;
 }
 
-// The public table's rule: what fl_attn_select_config reports, and the base
-// of select_d64, which launches by newer measurements where they differ (its
-// answers for given shapes are part of the interface; callers look them up).
+// The public table's rule: what fl_attn_select_config reports (its answers for
+// given shapes are part of the interface), and the base of select_d64, which
+// launches by newer measurements where they differ.
 //
 // Tile-configuration choice for the device's CUs (fl::device_cus(): 256 on
 // an MI355X seen whole, where the rules below were measured; every
@@ -297,6 +297,7 @@ struct KvPlan {
 };
 constexpr int kMaxSplits = 256;
 constexpr int64_t kPartFloats = 68;  // per row: O[64], m, l, 2 pad
+constexpr int64_t kPartFloats128 = 132;  // the same at head dim 128
 
 KvPlan plan_kvsplit(const fl::FwdArgs& a, int32_t requested) {
   const int64_t cus = fl::device_cus();
@@ -422,6 +423,23 @@ int select_d128(const fl::FwdArgs& a) {
   return fl::kSlotW4Config;
 }
 
+// The base rule of select_d64: fp16 follows the public rule; bf16 does where
+// that picks the streaming kernel, the key quarters, a key-range split or
+// block pairs, and otherwise takes a slot-scheduled group (4 waves for at most
+// 32 query rows over as many heads as CUs: 0-5% faster than 8).
+int select_base(const fl::FwdArgs& a) {
+  const int c = select_fa2(a);
+  if (a.dtype == fl::kDtypeF16 || c == fl::kCfgSplit2 || c == fl::kCfgSplit2W2 ||
+      c == fl::kCfgPair || c == fl::kCfgPairW2 || c == fl::kStreamConfig ||
+      c == fl::kQuarterConfig)
+    return c;
+  const int64_t cus = fl::device_cus();
+  if (a.seq <= 32 && a.batch_heads >= cus) return fl::kSlotW4Config;
+  const int64_t wgs256 = (a.seq + 255) / 256 * (int64_t)a.batch_heads;
+  return (!a.causal && a.seq_k >= 4096 && wgs256 >= cus) ? fl::kSlotW8Config
+                                                           : fl::kSlotW4Config;
+}
+
 // Head dim 64, fp16 and bf16 (sweeps of 1-1024 heads by N 40-8192, both
 // masks, us per call; fp16 figures, bf16 within 3% of them):
 //  - at most one 32-row block per CU, square causal 1.5 (their lengths
@@ -450,11 +468,8 @@ int select_d128(const fl::FwdArgs& a) {
 //  - fp16, non-causal from 2048 keys with more 256-row groups than CUs: those
 //    only from 4096 keys or where their last round is nearly full (B2 H16
 //    N3000, 1.5 rounds, 91.3 against 79.9 on the 4-wave groups).
-// Beyond these, fp16 follows the public rule; bf16 does where that picks the
-// streaming kernel, the key quarters, a key-range split or block pairs, and
-// otherwise takes a slot-scheduled group (4 waves for at most 32 query rows
-// over as many heads as CUs: 0-5% faster than 8).
-int select_d64(const fl::FwdArgs& a) {
+// Beyond these, the base rule.
+int select_d64_fast(const fl::FwdArgs& a) {
   const int64_t cus = fl::device_cus();
   auto wgs = [&](int64_t br) { return (a.seq + br - 1) / br * (int64_t)a.batch_heads; };
   const bool square = a.causal && a.seq == a.seq_k;
@@ -477,22 +492,86 @@ int select_d64(const fl::FwdArgs& a) {
   const int64_t pairs64 = (((int64_t)a.seq + 63) / 64 + 1) / 2 * a.batch_heads;
   if (square && a.seq_k >= 1792 && pairs64 <= cus) return fl::kCfgPairW2;
   if (!a.causal && a.seq_k >= 1280 && wgs(128) <= cus) return fl::kCfgSplit2;
-  const int c = select_fa2(a);
-  if (a.dtype == fl::kDtypeF16) {
-    const int64_t g = wgs(256), rounds = (g + cus - 1) / cus;
-    if (c == fl::kSlotW8Config && a.seq_k < 4096 && rounds > 1 && 10 * g < 9 * rounds * cus)
-      return fl::kSlotW4Config;
-    return c;
-  }
-  if (c == fl::kCfgSplit2 || c == fl::kCfgSplit2W2 || c == fl::kCfgPair || c == fl::kCfgPairW2 ||
-      c == fl::kStreamConfig || c == fl::kQuarterConfig)
-    return c;
-  return (!a.causal && a.seq_k >= 4096 && wgs(256) >= cus) ? fl::kSlotW8Config
-                                                            : fl::kSlotW4Config;
+  const int c = select_base(a);
+  const int64_t g = wgs(256), rounds = (g + cus - 1) / cus;
+  if (a.dtype == fl::kDtypeF16 && c == fl::kSlotW8Config && a.seq_k < 4096 && rounds > 1 &&
+      10 * g < 9 * rounds * cus)
+    return fl::kSlotW4Config;
+  return c;
+}
+
+// The log-sum-exp keeps its precision: the slot schedules sum the rounded p
+// (about 1e-5 of ln l), the other kernels the fp32 p, so a call that asks for
+// it and that the base rule gives one of those does not move to a slot
+// schedule.
+bool rounded_sums(int cfg) {
+  return cfg == fl::kCfgSplit2 || cfg == fl::kSlotW8Config || cfg == fl::kSlotW4Config ||
+         cfg == fl::kCfgSplit2W2 || cfg == fl::kCfgPair || cfg == fl::kCfgPairW2;
+}
+
+int select_d64(const fl::FwdArgs& a) {
+  const int c = select_d64_fast(a);
+  if (a.lse == nullptr || !rounded_sums(c)) return c;
+  const int base = select_base(a);
+  return rounded_sums(base) ? c : base;
 }
 
 int select_any(const fl::FwdArgs& a) {
   return a.head_dim == 128 ? select_d128(a) : select_d64(a);
+}
+
+// Split-KV plan of fl_attn_fwd_ws: fp16 at head_dim 64 follows plan_kvsplit;
+// the other types split at most 32 query rows per head into chunks of the
+// 32-row groups.  nsplit == 0: one pass.
+//
+// One query row in bf16, us per call, one pass against chunks (t: key tiles of
+// a head, 32 keys at head dim 128, 64 at 64).  The merge costs about 3 us, and
+// from half as many heads as CUs the one-pass groups fill the chip (128 heads
+// over 4096 keys at head dim 128: 52.2 against 51.6).  Up to one head per 8
+// CUs 8 chunks pay from 32 (24) tiles (16 heads: 1000 keys 9.3 against 8.0,
+// 4096 keys 24.1 against 11.7; at 600 keys 7.7 against 7.9; at head dim 64 1500
+// keys 8.6 against 7.3, 1000 keys 7.2 against 7.35), and long ranges take a
+// chunk per 16 tiles (2 heads over 16384 keys 13.3 with 16, 12.0 with 32).
+// More heads take about one chunk per CU, at least 4, from as many tiles as
+// heads, at most 64 (48 heads: 1500 keys 12.6 against 12.0, 1000 keys 10.0
+// against 10.7; 64 heads: 3000 keys 33.1 against 20.9; 100 heads over 4096
+// keys 51.2 against 41.9).
+struct WsPlan {
+  int nsplit;
+  int64_t bytes;
+  KvPlan kv;  // fp16 at head_dim 64
+};
+
+WsPlan plan_ws(const fl::FwdArgs& a) {
+  WsPlan p = {};
+  if (!narrow_configs(a)) {
+    p.kv = plan_kvsplit(a, 0);
+    p.nsplit = p.kv.nsplit;
+    p.bytes = p.kv.bytes;
+    return p;
+  }
+  const int64_t cus = fl::device_cus(), heads = a.batch_heads;
+  const int64_t keys = a.head_dim == 64 ? 64 : 32;
+  const int64_t tiles = (a.seq_k + keys - 1) / keys;
+  const int64_t row = a.head_dim == 64 ? kPartFloats : kPartFloats128;
+  if (a.seq > 32 || 2 * heads >= cus) return p;
+  int64_t n, least;
+  if (8 * heads <= cus) {
+    n = std::min(std::max<int64_t>(8, tiles / 16), 2 * cus / heads);
+    least = a.head_dim == 64 ? 24 : 32;
+  } else {
+    n = std::max<int64_t>(4, cus / heads);
+    least = std::min<int64_t>(heads, 64);
+  }
+  if (tiles < least) return p;
+  p.nsplit = (int)std::min<int64_t>(n, kMaxSplits);
+  p.bytes = p.nsplit * heads * a.seq * row * (int64_t)sizeof(float);
+  return p;
+}
+
+hipError_t run_ws(const fl::FwdArgs& a, const WsPlan& p, float* part, hipStream_t st) {
+  return narrow_configs(a) ? fl::launch_kvsplit_rows32(a, part, p.nsplit, st)
+                           : run_kvsplit(a, p.kv, part, st);
 }
 
 int fwd_ex(const fl_attn_params_ex* p, int32_t config, void* stream, int dtype, const char* who) {
@@ -620,6 +699,40 @@ int fl_attn_fwd_f16_ex(const fl_attn_params_ex* p, int32_t config, void* stream)
 
 int fl_attn_fwd_bf16_ex(const fl_attn_params_ex* p, int32_t config, void* stream) {
   return fwd_ex(p, config, stream, fl::kDtypeBF16, "fl_attn_fwd_bf16_ex");
+}
+
+int64_t fl_attn_workspace_bytes(const fl_attn_params_ex* p, int32_t dtype) {
+  const char* who = "fl_attn_workspace_bytes";
+  fl::FwdArgs a;
+  if (dtype != FL_DTYPE_F16 && dtype != FL_DTYPE_BF16)
+    return fail(FL_ERR_INVALID_ARGUMENT, "%s: unknown dtype %d", who, (int)dtype), -1;
+  if (check_ex(p, &a, who, /*wide=*/true) != FL_OK) return -1;
+  a.dtype = dtype == FL_DTYPE_BF16 ? fl::kDtypeBF16 : fl::kDtypeF16;
+  if (empty_problem(a)) return 0;
+  return plan_ws(a).bytes;
+}
+
+int fl_attn_fwd_ws(const fl_attn_params_ex* p, int32_t dtype, void* workspace,
+                   int64_t workspace_bytes, void* stream) {
+  const char* who = "fl_attn_fwd_ws";
+  fl::FwdArgs a;
+  if (dtype != FL_DTYPE_F16 && dtype != FL_DTYPE_BF16)
+    return fail(FL_ERR_INVALID_ARGUMENT, "%s: unknown dtype %d", who, (int)dtype);
+  int rc = check_ex(p, &a, who, /*wide=*/true);
+  if (rc != FL_OK) return rc;
+  a.dtype = dtype == FL_DTYPE_BF16 ? fl::kDtypeBF16 : fl::kDtypeF16;
+  if (empty_problem(a)) return FL_OK;
+  rc = check_pointers(&p->base, &a, who, 16);
+  if (rc != FL_OK) return rc;
+  const WsPlan plan = plan_ws(a);
+  const bool split = plan.nsplit != 0 && workspace != nullptr && workspace_bytes >= plan.bytes;
+  if (split && ((uintptr_t)workspace & 15))
+    return fail(FL_ERR_MISALIGNED, "%s: workspace must be 16-byte aligned", who);
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  const hipError_t e = split ? run_ws(a, plan, static_cast<float*>(workspace), st)
+                             : fl::launch_fa2(a, select_any(a), st);
+  if (e != hipSuccess) return fail(FL_ERR_LAUNCH, "%s: launch failed: %s", who, hipGetErrorString(e));
+  return FL_OK;
 }
 
 int64_t fl_attn_splitkv_workspace_bytes(const fl_attn_params_ex* p, int32_t num_splits) {

@@ -185,6 +185,7 @@ struct Geom {
 // Floats per row of a split-KV partial result: O[64] unnormalised, the
 // stabiliser in base-2 logit units, the row sum, 2 pad (16-byte rows).
 constexpr int kPartStride = 68;
+constexpr int kPartStride128 = 132;  // the same at head dim 128
 
 // Per-head base pointers and buffer resources of a work-group.
 template <class T = _Float16>
@@ -310,6 +311,22 @@ __device__ __forceinline__ void pair_coords(int nqb, int xcds, int& bh, int& p) 
   const int lin = per * xcds == total ? (i % xcds) * per + i / xcds : i;
   bh = lin / np;
   p = lin - bh * np;
+}
+
+// Work-group -> (batch*head, key chunk, query block) of a split-KV launch:
+// the query blocks of one chunk, which read the same K and V, are
+// consecutive, and consecutive work-groups of an XCD stay together when they
+// divide evenly.
+__device__ __forceinline__ void chunk_coords(int nqb, int nsplit, int xcds, int& bh, int& chunk,
+                                             int& qb) {
+  const int total = gridDim.x;
+  const int i = blockIdx.x;
+  const int per = total / xcds;
+  const int lin = per * xcds == total ? (i % xcds) * per + i / xcds : i;
+  const int c = lin / nqb;
+  qb = lin - c * nqb;
+  bh = c / nsplit;
+  chunk = c - bh * nsplit;
 }
 
 // Asynchronous fetch of tile t (clamped to the last tile the work-group

@@ -208,12 +208,17 @@ fa2_fwd_kernel(const _Float16* Q, const _Float16* __restrict__ K,
 // Split-KV combine: one wave per query row merges the nsplit partials of the
 // row (O unnormalised at stabiliser m_s, row sum l_s) at their largest m:
 //   O = sum_s 2^(m_s - M) O_s / sum_s 2^(m_s - M) l_s,
-// and writes O (fp16, lane = head dim) and, when asked, the log-sum-exp.
-// Lane j holds m and l of chunks j, j + 64, ...; its weight w_j goes to the
-// whole wave by readlane, and each batch of 8 chunks issues its 8 O loads
-// before the first multiply, so the row costs a few memory round trips
-// rather than one per chunk.  A chunk with no visible key stored m = -inf
-// and l = 0: weight 0, skipped by a select, not a branch.
+// and writes O (lane = head dim, or two of them at head dim 128) and, when
+// asked, the log-sum-exp.  Lane j holds m and l of chunks j, j + 64, ...; its
+// weight w_j goes to the whole wave by readlane.  The row is bound by memory
+// round trips.  Up to 24 chunks, m, l and every O leave together: no O load
+// waits for a weight (B1 H8 N_q 1 N_k 3000, 6 chunks: 9.65 -> 8.3 us a call,
+// chunk kernel included; B2 H8 N_k 4096, 8 chunks: 9.2 -> 8.7; B1 H16
+// N_q 4 N_k 8192, 16 chunks: 12.2 -> 11.5).  Beyond, each
+// batch of 8 chunks issues its O loads before the first multiply; up-front
+// batches there measured up to 15% slower (128 and more chunks).  A chunk with
+// no visible key stored m = -inf and l = 0: weight 0, skipped by a select, not
+// a branch.
 __device__ __forceinline__ float wave_max64(float x) {
 #pragma unroll
   for (int m = 32; m >= 1; m >>= 1) x = fmaxf(x, __shfl_xor(x, m, 64));
@@ -226,48 +231,86 @@ __device__ __forceinline__ float wave_sum64(float x) {
   return x;
 }
 
+template <int D, class T>
 __global__ void __launch_bounds__(256)
-splitkv_combine_kernel(_Float16* O, const Geom geom) {
+splitkv_combine_kernel(T* O, const Geom geom) {
+  constexpr int kPart = D == 64 ? kPartStride : kPartStride128;
+  constexpr int kCols = D / 64;  // head dims lane, lane + 64
+  constexpr int kBatch = 8, kUpFront = 3;  // chunks per batch, batches loaded up front
   const int lane = threadIdx.x & 63;
   const int row_id = blockIdx.x * 4 + (threadIdx.x >> 6);  // bh * N_q + row
   if (row_id >= geom.batch_heads * geom.seq_q) return;
   const int bh = row_id / geom.seq_q, row = row_id - bh * geom.seq_q;
-  const long long split_stride = (long long)geom.batch_heads * geom.seq_q * kPartStride;
-  const float* p0 = geom.part + (long long)row_id * kPartStride;
+  const long long split_stride = (long long)geom.batch_heads * geom.seq_q * kPart;
+  const float* p0 = geom.part + (long long)row_id * kPart;
   const int ns = geom.nsplit;
-  float mx = ninf();
-  for (int s = lane; s < ns; s += 64) mx = fmaxf(mx, p0[s * split_stride + 64]);
-  mx = wave_max64(mx);
-  float acc = 0.0f, lpart = 0.0f;
-  for (int s0 = 0; s0 < ns; s0 += 64) {
-    float w = 0.0f;
-    if (s0 + lane < ns) {
-      const float* ps = p0 + (s0 + lane) * split_stride;
-      const float m = ps[64];
-      w = m == ninf() ? 0.0f : __builtin_amdgcn_exp2f(m - mx);
-      lpart += w * ps[65];
-    }
-    // Chunk s0 + j's weight, from lane j; a weight of 0 skips the chunk.
-    auto fold = [&](int j, float oj) __attribute__((always_inline)) {
-      const float wj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), j));
-      acc += wj == 0.0f ? 0.0f : wj * oj;
-    };
-    const int cnt = min(64, ns - s0);
-    const float* pb = p0 + (long long)s0 * split_stride + lane;
-    int j = 0;
-    for (; j + 8 <= cnt; j += 8) {
-      float o[8];
+  float acc[kCols] = {}, lpart = 0.0f, mx;
+  // Chunk s0 + j's weight, from lane j of w; a weight of 0 skips the chunk.
+  auto fold = [&](float w, int j, const float (&x)[kCols]) __attribute__((always_inline)) {
+    const float wj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), j));
 #pragma unroll
-      for (int u = 0; u < 8; ++u) o[u] = pb[(j + u) * split_stride];
+    for (int c = 0; c < kCols; ++c) acc[c] += wj == 0.0f ? 0.0f : wj * x[c];
+  };
+  auto load = [&](int s, float (&x)[kCols]) __attribute__((always_inline)) {
 #pragma unroll
-      for (int u = 0; u < 8; ++u) fold(j + u, o[u]);
+    for (int c = 0; c < kCols; ++c) x[c] = p0[s * split_stride + lane + 64 * c];
+  };
+  if (ns <= kUpFront * kBatch) {
+    float m = ninf(), l = 0.0f;
+    if (lane < ns) {
+      m = p0[lane * split_stride + D];
+      l = p0[lane * split_stride + D + 1];
     }
-    for (; j < cnt; ++j) fold(j, pb[j * split_stride]);
+    // (past the last chunk: its values again, weight 0)
+    float o[kUpFront][kBatch][kCols];
+#pragma unroll
+    for (int i = 0; i < kUpFront; ++i)
+      if (i == 0 || ns > i * kBatch) {
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u) load(min(i * kBatch + u, ns - 1), o[i][u]);
+      }
+    mx = wave_max64(m);
+    const float w = m == ninf() ? 0.0f : __builtin_amdgcn_exp2f(m - mx);
+    lpart = w * l;
+#pragma unroll
+    for (int i = 0; i < kUpFront; ++i)
+      if (i == 0 || ns > i * kBatch) {
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u) fold(w, i * kBatch + u, o[i][u]);
+      }
+  } else {
+    mx = ninf();
+    for (int s = lane; s < ns; s += 64) mx = fmaxf(mx, p0[s * split_stride + D]);
+    mx = wave_max64(mx);
+    for (int s0 = 0; s0 < ns; s0 += 64) {
+      float w = 0.0f;
+      if (s0 + lane < ns) {
+        const float m = p0[(s0 + lane) * split_stride + D];
+        w = m == ninf() ? 0.0f : __builtin_amdgcn_exp2f(m - mx);
+        lpart += w * p0[(s0 + lane) * split_stride + D + 1];
+      }
+      const int cnt = min(64, ns - s0);
+      int j = 0;
+      for (; j + kBatch <= cnt; j += kBatch) {
+        float o[kBatch][kCols];
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u) load(s0 + j + u, o[u]);
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u) fold(w, j + u, o[u]);
+      }
+      for (; j < cnt; ++j) {
+        float o[kCols];
+        load(s0 + j, o);
+        fold(w, j, o);
+      }
+    }
   }
   const float lsum = wave_sum64(lpart);
   const int b = bh / geom.heads, h = bh - b * geom.heads;
-  _Float16* orow = O + (b * geom.o_sb + h * geom.o_sh) + (long long)row * geom.o_sr;
-  orow[lane] = (_Float16)(lsum > 0.0f ? acc / lsum : 0.0f);
+  T* orow = O + (b * geom.o_sb + h * geom.o_sh) + (long long)row * geom.o_sr;
+#pragma unroll
+  for (int c = 0; c < kCols; ++c)
+    orow[lane + 64 * c] = (T)(lsum > 0.0f ? acc[c] / lsum : 0.0f);
   if (geom.lse != nullptr && lane == 0)
     geom.lse[row_id] =
         lsum > 0.0f ? 0.693147180559945309f * (mx + __builtin_amdgcn_logf(lsum)) : ninf();
@@ -328,8 +371,22 @@ hipError_t launch_splitkv_combine(const FwdArgs& a, float* part, int nsplit, hip
   g.part = part;
   g.nsplit = nsplit;
   const int rows = a.batch_heads * a.seq;
-  hipLaunchKernelGGL(splitkv_combine_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, st,
-                     static_cast<_Float16*>(a.o), g);
+  const dim3 grid((unsigned)((rows + 3) / 4)), block(256);
+  const bool bf = a.dtype == kDtypeBF16;
+  if (a.head_dim == 128) {
+    if (bf)
+      hipLaunchKernelGGL((splitkv_combine_kernel<128, __bf16>), grid, block, 0, st,
+                         static_cast<__bf16*>(a.o), g);
+    else
+      hipLaunchKernelGGL((splitkv_combine_kernel<128, _Float16>), grid, block, 0, st,
+                         static_cast<_Float16*>(a.o), g);
+  } else if (bf) {
+    hipLaunchKernelGGL((splitkv_combine_kernel<64, __bf16>), grid, block, 0, st,
+                       static_cast<__bf16*>(a.o), g);
+  } else {
+    hipLaunchKernelGGL((splitkv_combine_kernel<64, _Float16>), grid, block, 0, st,
+                       static_cast<_Float16*>(a.o), g);
+  }
   return hipGetLastError();
 }
 

@@ -90,7 +90,7 @@ struct TileRows<64, T, CAUSAL> : Rows<CAUSAL, true, T> {
   __device__ __forceinline__ float stabiliser() const { return this->m * this->cr; }
 };
 
-template <int D, int NW, bool CAUSAL, class T>
+template <int D, int NW, bool CAUSAL, class T, bool KVSPLIT>
 __global__ void __launch_bounds__(64 * NW, 2)
 fa2_fwd_rows32_kernel(const T* Q, const T* __restrict__ K, const T* __restrict__ V, T* O,
                       const Geom geom, int nqb, float cq, float cr) {
@@ -108,18 +108,28 @@ fa2_fwd_rows32_kernel(const T* Q, const T* __restrict__ K, const T* __restrict__
 
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  int bh, qb;
-  wg_coords<false, 1>(nqb, geom.xcds, geom.cus_per_xcd, bh, qb);
+  int bh, qb, chunk = 0;
+  if constexpr (KVSPLIT)
+    chunk_coords(nqb, geom.nsplit, geom.xcds, bh, chunk, qb);
+  else
+    wg_coords<false, 1>(nqb, geom.xcds, geom.cus_per_xcd, bh, qb);
   const HeadPtrs<T> hp = head_ptrs<T, kRowB>(geom, bh, Q, K, V, O);
   const int seq = geom.seq_q, q0 = 32 * qb;
-  // The block's key tiles (through its last row's diagonal), of which this
-  // wave takes w + NW i, i < n.
-  int tiles = max(1, (geom.seq_k + kKeys - 1) / kKeys);
+  // The group's key tiles [tbeg, tiles), through its last row's diagonal and
+  // its chunk's end; this wave takes tbeg + w + NW i, i < n (none in a chunk
+  // past the diagonal).
+  int tiles = max(1, (geom.seq_k + kKeys - 1) / kKeys), tbeg = 0;
+  if constexpr (KVSPLIT) {
+    const int per = (tiles + geom.nsplit - 1) / geom.nsplit;
+    tbeg = chunk * per;
+    tiles = min(tiles, tbeg + per);
+  }
   if (CAUSAL) {
     const int last_key = min(q0 + 32, seq) - 1 + geom.coff;
     tiles = min(tiles, last_key < 0 ? 1 : last_key / kKeys + 1);
   }
-  const int n = tiles > w ? (tiles - w + NW - 1) / NW : 0;
+  const int mine0 = tbeg + w;  // this wave's first tile
+  const int n = tiles > mine0 ? (tiles - mine0 + NW - 1) / NW : 0;
 
   const FetchOff<8> fk = D == 64 ? fetch_offsets<8, false>(0, lane, 2 * geom.k_sr)
                                  : fetch_offsets128<8, false>(0, lane, 2 * geom.k_sr);
@@ -128,10 +138,10 @@ fa2_fwd_rows32_kernel(const T* Q, const T* __restrict__ K, const T* __restrict__
   i32x4_t rk, rv;
   kv_rsrc_rows<T, kRowB>(geom, bh, K, V, tiles * kKeys, rk, rv);
   auto fetch_k = [&](int i) __attribute__((always_inline)) {
-    fetch_tile_z<8>(rk, buf[w][0], w + NW * i, tiles, 0, fk);
+    fetch_tile_z<8>(rk, buf[w][0], mine0 + NW * i, tiles, 0, fk);
   };
   auto fetch_v = [&](int i) __attribute__((always_inline)) {
-    fetch_tile_z<8>(rv, buf[w][1], w + NW * i, tiles, 0, fv);
+    fetch_tile_z<8>(rv, buf[w][1], mine0 + NW * i, tiles, 0, fv);
   };
   // A part of the block's Q first (its wait leaves the tiles in flight).
   if constexpr (D == 64)
@@ -151,7 +161,7 @@ fa2_fwd_rows32_kernel(const T* Q, const T* __restrict__ K, const T* __restrict__
     rows.scores(buf[w][0], s);
     asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");  // its operands are in registers
     fetch_k(i + 1);
-    rows.softmax(w + NW * i, i == 0, s, p);
+    rows.softmax(mine0 + NW * i, i == 0, s, p);
     asm volatile("s_waitcnt vmcnt(8)" : : : "memory");  // V(i)
     rows.output(buf[w][1], p);
     asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
@@ -186,6 +196,10 @@ fa2_fwd_rows32_kernel(const T* Q, const T* __restrict__ K, const T* __restrict__
   const float l_tot = pair_sum(lt);
   const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
   const bool mine_row = rows.my_q < seq;
+  constexpr int kPart = D == 64 ? kPartStride : kPartStride128;
+  float* const prow = KVSPLIT ? geom.part + ((long long)(chunk * geom.batch_heads + bh) * seq +
+                                             rows.my_q) * kPart
+                              : nullptr;
   for (int c = w; c < D / 16; c += NW) {
     // 8-column piece c of the row: accumulators 8 (c & 1) .. + 7 of block c / 2
     float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -203,37 +217,48 @@ fa2_fwd_rows32_kernel(const T* Q, const T* __restrict__ K, const T* __restrict__
       acc[7] += a[j] * x1.w;
     }
     const int col = 32 * (c >> 1) + 16 * (c & 1) + 8 * rows.g;
-    if (mine_row) {
+    if (!mine_row) continue;
+    if constexpr (KVSPLIT) {
+      *reinterpret_cast<float4*>(prow + col) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+      *reinterpret_cast<float4*>(prow + col + 4) = make_float4(acc[4], acc[5], acc[6], acc[7]);
+    } else {
       V8 out;
 #pragma unroll
       for (int e = 0; e < 8; ++e) out[e] = (T)(acc[e] * inv);
       *reinterpret_cast<V8*>(hp.o + (long long)rows.my_q * geom.o_sr + col) = out;
     }
   }
-  if (w == 0 && rows.g == 0 && mine_row && hp.lse != nullptr)
+  if (w != 0 || rows.g != 0 || !mine_row) return;
+  if constexpr (KVSPLIT) {
+    prow[D] = l_tot > 0.0f ? mm : ninf();
+    prow[D + 1] = l_tot;
+  } else if (hp.lse != nullptr) {
     hp.lse[rows.my_q] =
         l_tot > 0.0f ? 0.693147180559945309f * (mm + __builtin_amdgcn_logf(l_tot)) : ninf();
+  }
 }
 
 // Eight waves for blocks of at least 32 tiles at head dim 64, where they fit
 // one round (B1 H1 N2048 9.2 against 9.7 us with four, N4096 13.5 against
 // 15.1; N1024 equal, shorter ones up to 10% slower; at head dim 128 0-8%
 // slower but for a tie at B1 H2 N2048).
-template <int D, class T>
-hipError_t launch_rows32_t(const FwdArgs& a, hipStream_t st) {
+template <int D, class T, bool KVSPLIT>
+hipError_t launch_rows32_t(const FwdArgs& a, float* part, int nsplit, hipStream_t st) {
   const int nqb = (a.seq + 31) / 32;
   const Scales sc(a);
-  const Geom g = make_geom(a);
-  const unsigned groups = (unsigned)(nqb * a.batch_heads);
+  Geom g = make_geom(a);
+  g.part = part;
+  g.nsplit = nsplit;
+  const unsigned groups = (unsigned)(nqb * a.batch_heads * nsplit);
   const T *q = static_cast<const T*>(a.q), *k = static_cast<const T*>(a.k),
           *v = static_cast<const T*>(a.v);
   T* o = static_cast<T*>(a.o);
   auto go = [&](auto nw, auto causal) {
     constexpr int NW = decltype(nw)::value;
-    hipLaunchKernelGGL((fa2_fwd_rows32_kernel<D, NW, decltype(causal)::value != 0, T>),
+    hipLaunchKernelGGL((fa2_fwd_rows32_kernel<D, NW, decltype(causal)::value != 0, T, KVSPLIT>),
                        dim3(groups), dim3(64 * NW), 0, st, q, k, v, o, g, nqb, sc.cq, sc.cr);
   };
-  if constexpr (D == 64) {
+  if constexpr (D == 64 && !KVSPLIT) {
     if (a.seq_k >= 2048 && groups <= (unsigned)device_cus()) {
       a.causal ? go(Ic<8>{}, Ic<1>{}) : go(Ic<8>{}, Ic<0>{});
       return hipGetLastError();
@@ -243,13 +268,25 @@ hipError_t launch_rows32_t(const FwdArgs& a, hipStream_t st) {
   return hipGetLastError();
 }
 
+template <bool KVSPLIT>
+hipError_t launch_rows32_any(const FwdArgs& a, float* part, int nsplit, hipStream_t st) {
+  const bool bf = a.dtype == kDtypeBF16;
+  if (a.head_dim == 128)
+    return bf ? launch_rows32_t<128, __bf16, KVSPLIT>(a, part, nsplit, st)
+              : launch_rows32_t<128, _Float16, KVSPLIT>(a, part, nsplit, st);
+  return bf ? launch_rows32_t<64, __bf16, KVSPLIT>(a, part, nsplit, st)
+            : launch_rows32_t<64, _Float16, KVSPLIT>(a, part, nsplit, st);
+}
+
 }  // namespace
 
 hipError_t launch_rows32(const FwdArgs& a, hipStream_t st) {
-  const bool bf = a.dtype == kDtypeBF16;
-  if (a.head_dim == 128)
-    return bf ? launch_rows32_t<128, __bf16>(a, st) : launch_rows32_t<128, _Float16>(a, st);
-  return bf ? launch_rows32_t<64, __bf16>(a, st) : launch_rows32_t<64, _Float16>(a, st);
+  return launch_rows32_any<false>(a, nullptr, 1, st);
+}
+
+hipError_t launch_kvsplit_rows32(const FwdArgs& a, float* part, int nsplit, hipStream_t st) {
+  const hipError_t e = launch_rows32_any<true>(a, part, nsplit, st);
+  return e != hipSuccess ? e : launch_splitkv_combine(a, part, nsplit, st);
 }
 
 }  // namespace fl

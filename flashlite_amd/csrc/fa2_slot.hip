@@ -287,7 +287,10 @@ fa2_fwd_slot_kernel(const T* Q, const T* __restrict__ K, const T* __restrict__ V
       else
         fetch_seg<kSegs>(rv, rings.vslot(Ic<I + FV>{}), tbv, d - kSegs, rw, fv);
     };
-    if constexpr (!kSpread) static_for(std::make_integer_sequence<int, kDmaPerIter>{}, fetch);
+    if constexpr (!kSpread) {
+      fetch_tile_z<kSegs>(rk, rings.kslot(Ic<I + FK>{}), tbeg + j + FK, tzero, rw, fk);
+      fetch_tile_z<kSegs>(rv, rings.vslot(Ic<I + FV>{}), tbeg + j + FV, tzero, rw, fv);
+    }
     V8 op[16];
     V8 top[kLastTail];  // kLast: the tail MFMAs' operands
 #pragma unroll

@@ -138,6 +138,9 @@ hipError_t launch_kvsplit(const FwdArgs& a, int waves, float* part, int nsplit,
 // The same with single-wave query blocks (N_q <= 32) in key-quarter chunks
 // of at most kQuarterMaxKeys keys: 4 waves per chunk (fa2_short.hip).
 hipError_t launch_kvsplit_quarter(const FwdArgs& a, float* part, int nsplit, hipStream_t stream);
+// The same in chunks of the 32-row groups, any element type and head dim
+// (at head dim 128 the partials are 132 floats a row; fa2_rows32.hip).
+hipError_t launch_kvsplit_rows32(const FwdArgs& a, float* part, int nsplit, hipStream_t stream);
 // The combine kernel alone (fa2_pipe.hip): merges the nsplit partials in
 // `part` into O (and the log-sum-exp when a.lse is set).
 hipError_t launch_splitkv_combine(const FwdArgs& a, float* part, int nsplit, hipStream_t stream);

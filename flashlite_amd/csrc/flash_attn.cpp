@@ -54,6 +54,25 @@ void check_same_device(const torch::Tensor& q, const torch::Tensor& k, const tor
               "All tensors must be on the same device");
 }
 
+// bf16 and head_dim 128 (`wide`) calls took any `workspace` without looking at
+// it while they ran one pass only: one they cannot use is still no error.
+bool usable_workspace(const torch::Tensor& ws, const torch::Tensor& q) {
+  return ws.is_cuda() && ws.device() == q.device() && ws.is_contiguous() &&
+         reinterpret_cast<uintptr_t>(ws.data_ptr()) % 16 == 0;
+}
+
+// A wide call with `out` given allocated nothing, so it could be captured by
+// means the caching allocator does not see; under capture it still allocates
+// nothing.
+bool capturing(void* stream) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(static_cast<hipStream_t>(stream), &st) != hipSuccess) {
+    (void)hipGetLastError();  // not the next launch's error
+    return false;
+  }
+  return st != hipStreamCaptureStatusNone;
+}
+
 }  // namespace
 
 torch::Tensor flash_attn_forward_naive(torch::Tensor q, torch::Tensor k, torch::Tensor v,
@@ -139,7 +158,8 @@ torch::Tensor flash_attn_forward_flash2(torch::Tensor q, torch::Tensor k, torch:
 // q's layout (empty_like keeps dense strides); an omitted `lse` (with
 // return_lse) as a contiguous fp32 [B, H, N_q] tensor.  Passing both keeps
 // the call free of allocations (apart from a split-KV workspace, see below).
-// num_splits: 0 = the library's choice, 1 = one pass, n > 1 = n key chunks.
+// num_splits: 0 = the library's choice, 1 = one pass, n > 1 = n key chunks
+// (fp16 at head_dim 64).
 // A split-KV call needs a workspace: `workspace` (any device tensor of
 // enough bytes, reused across calls for an allocation-free loop) or else
 // one from the caching allocator.
@@ -204,12 +224,15 @@ py::object flash_attn_forward_flash2_ex(torch::Tensor q, torch::Tensor k, torch:
     for (int d = 0; d < 3; ++d) st[i][d] = ts[i]->stride(d);
   p.lse = return_lse ? lse.data_ptr<float>() : nullptr;
   TORCH_CHECK(num_splits >= 0 && num_splits <= INT32_MAX, "num_splits must be >= 0");
-  // Split-KV is built for fp16 at head_dim 64; bf16 and head_dim 128 run one pass.
-  const bool one_pass_only = bf16 || head_dim != 64;
-  TORCH_CHECK(!one_pass_only || num_splits <= 1,
+  // An explicit chunk count is built for fp16 at head_dim 64; with
+  // num_splits 0 the library chooses for every type.
+  const bool wide = bf16 || head_dim != 64;
+  TORCH_CHECK(!wide || num_splits <= 1,
               "split-KV (num_splits > 1) needs fp16 tensors with head_dim 64");
-  const int64_t ws_bytes = (num_splits == 1 || one_pass_only)
-                               ? 0
+  const int32_t dtype = bf16 ? FL_DTYPE_BF16 : FL_DTYPE_F16;
+  const int64_t ws_bytes = num_splits == 1 ? 0
+                           : num_splits == 0
+                               ? fl_attn_workspace_bytes(&p, dtype)
                                : fl_attn_splitkv_workspace_bytes(&p, (int32_t)num_splits);
   TORCH_CHECK(ws_bytes >= 0, "FlashLite HIP error: ", fl_attn_last_error());
   int rc;
@@ -218,16 +241,24 @@ py::object flash_attn_forward_flash2_ex(torch::Tensor q, torch::Tensor k, torch:
               : fl_attn_fwd_f16_ex(&p, -1, current_stream(q));
   } else {
     torch::Tensor ws;
+    void* buf = nullptr;
+    size_t have = 0;
     if (workspace.has_value() && workspace.value().defined() &&
-        workspace.value().nbytes() >= (size_t)ws_bytes) {
+        workspace.value().nbytes() >= (size_t)ws_bytes &&
+        (!wide || usable_workspace(workspace.value(), q))) {
       ws = workspace.value();
       TORCH_CHECK(ws.is_cuda() && ws.device() == q.device() && ws.is_contiguous(),
                   "workspace must be a contiguous tensor on q's device");
-    } else {
+      buf = ws.data_ptr();
+      have = ws.nbytes();
+    } else if (!wide || !capturing(current_stream(q))) {
       ws = torch::empty({(ws_bytes + 3) / 4}, q.options().dtype(torch::kFloat32));
-    }
-    rc = fl_attn_fwd_f16_splitkv(&p, (int32_t)num_splits, ws.data_ptr(), (int64_t)ws.nbytes(),
-                                 current_stream(q));
+      buf = ws.data_ptr();
+      have = ws.nbytes();
+    }  // a wide call under capture without a workspace: one pass, nothing allocated
+    rc = num_splits == 0 ? fl_attn_fwd_ws(&p, dtype, buf, (int64_t)have, current_stream(q))
+                         : fl_attn_fwd_f16_splitkv(&p, (int32_t)num_splits, buf, (int64_t)have,
+                                                   current_stream(q));
   }
   TORCH_CHECK(rc == FL_OK, "FlashLite HIP error: ", fl_attn_last_error());
   if (return_lse) return py::make_tuple(out_tensor, lse);
@@ -266,8 +297,15 @@ PYBIND11_MODULE(flash_attn_wmma, m) {
             p.k_stride[d] = p.v_stride[d] = ks[d];
           }
           p.lse = nullptr;
-          if (num_splits == 1 || q.scalar_type() != torch::kHalf || q.size(3) != 64)
-            return (int64_t)0;  // one pass: split-KV is built for fp16 at head_dim 64
+          if (num_splits == 1) return (int64_t)0;
+          const bool bf16 = q.scalar_type() == torch::kBFloat16;
+          if (q.scalar_type() != torch::kHalf || q.size(3) != 64) {
+            // bf16 and head_dim 128 split by the library's choice only; what
+            // forward_flash2_ex will refuse needs no workspace
+            if (num_splits != 0 || (!bf16 && q.scalar_type() != torch::kHalf)) return (int64_t)0;
+            const int64_t w = fl_attn_workspace_bytes(&p, bf16 ? FL_DTYPE_BF16 : FL_DTYPE_F16);
+            return w > 0 ? w : (int64_t)0;
+          }
           const int64_t b = fl_attn_splitkv_workspace_bytes(&p, (int32_t)num_splits);
           TORCH_CHECK(b >= 0, "FlashLite HIP error: ", fl_attn_last_error());
           return b;

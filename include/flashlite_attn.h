@@ -134,6 +134,25 @@ int fl_attn_fwd_f16_ex(const fl_attn_params_ex* p, int32_t config, void* stream)
 int fl_attn_fwd_bf16_ex(const fl_attn_params_ex* p, int32_t config, void* stream);
 
 /*
+ * The dispatcher's choice for either element type (FL_DTYPE_*) and head_dim
+ * (64 or 128), with split-KV where it pays: as fl_attn_fwd_f16_ex /
+ * fl_attn_fwd_bf16_ex with config -1, but a problem with few query rows over
+ * many keys cuts its key range into chunks whose partial results go to
+ * `workspace` and are merged by a second kernel on the same stream.
+ * fl_attn_workspace_bytes returns the bytes such a call uses (0: one pass,
+ * -1: `p` is rejected).  With less (or a NULL workspace) the call runs one
+ * pass.  The workspace is 16-byte aligned device memory owned by the caller;
+ * calls that may overlap must not share one.
+ *
+ * No counterpart in the reference.
+ */
+#define FL_DTYPE_F16 0
+#define FL_DTYPE_BF16 1
+int64_t fl_attn_workspace_bytes(const fl_attn_params_ex* p, int32_t dtype);
+int fl_attn_fwd_ws(const fl_attn_params_ex* p, int32_t dtype, void* workspace,
+                   int64_t workspace_bytes, void* stream);
+
+/*
  * Split-KV forward ("flash-decoding"), fp16 at head_dim 64, for few query
  * rows over many keys:
  * the key range of every (batch, head) is cut into chunks processed by

@@ -61,3 +61,20 @@ def test_no_keys(cuda, kind, d):
     empty = np.zeros((1, 2, 0, d), dtype=np.float32)
     out, lse = run_wide(kind, q, empty, empty, 0.1, False, cuda, lse=True)
     assert (out == 0).all() and np.isneginf(lse).all()
+
+
+@pytest.mark.parametrize("kind", ["fp16", "bf16"])
+@pytest.mark.parametrize("h,nq,nk", [(512, 16, 455), (300, 100, 97), (100, 130, 200)])
+def test_lse_sums_stay_fp32(cuda, kind, h, nq, nk):
+    """Key ranges of at most 512 keys sum the unrounded p for the log-sum-exp
+    whatever schedule serves the call without it: fp32 rounding of the scores
+    and the sum (2^-24 of |lse| ~ 6 and of nk terms), against 2^-12 and more
+    for sums of rounded p."""
+    q, k, v = wide_inputs(kind, 1, h, nq, nk, 64, seed=h + nk)
+    out, lse = run_wide(kind, q, k, v, 0.125, False, cuda, lse=True)
+    mx, mean = wide_tol(kind)
+    ref = attention_fp32(q, k, v, 0.125, False)
+    assert_close_oracle(out, None, None, None, 0.125, False, max_abs=mx, mean_abs=mean, ref=ref)
+    assert error_stats(lse, attention_lse(q, k, 0.125, False))[0] <= 1e-5
+    out, _ = run_wide(kind, q, k, v, 0.125, False, cuda)
+    assert_close_oracle(out, None, None, None, 0.125, False, max_abs=mx, mean_abs=mean, ref=ref)
