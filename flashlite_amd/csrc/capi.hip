@@ -555,6 +555,8 @@ WsPlan plan_ws(const fl::FwdArgs& a) {
   const int64_t tiles = (a.seq_k + keys - 1) / keys;
   const int64_t row = a.head_dim == 64 ? kPartFloats : kPartFloats128;
   if (a.seq > 32 || 2 * heads >= cus) return p;
+  // the 32-row groups' buffer offsets within a Q block (fetch_q_block)
+  if (a.head_dim == 64 && a.q_sr > (1 << 24)) return p;
   int64_t n, least;
   if (8 * heads <= cus) {
     n = std::min(std::max<int64_t>(8, tiles / 16), 2 * cus / heads);

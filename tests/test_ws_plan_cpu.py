@@ -38,6 +38,17 @@ def test_fp16_d64_follows_the_split_plan():
         assert capi.workspace_bytes(p, capi.DTYPE_F16) == capi.splitkv_workspace_bytes(p, 0)
 
 
+def test_wide_query_row_strides():
+    # at head dim 64 a chunk's Q rows must lie within 32-bit byte offsets
+    for d, splits in ((64, False), (128, True)):
+        base = capi.make_params(0x10000, 0x20000, 0x30000, 0x40000, 1, 16, 16, 4096, d, 0.1, False)
+        ks = (16 * 4096 * d, 4096 * d, d)
+        for row, want in ((1 << 24, True), ((1 << 24) + 8, splits), (1 << 27, splits)):
+            qs = (16 * d, d, row)
+            p = capi.make_params_ex(base, qs, ks, ks, qs)
+            assert (capi.workspace_bytes(p, capi.DTYPE_BF16) > 0) == want
+
+
 def test_refusals():
     assert need(2, 64, 4, 1, 4096) == -1
     assert need(capi.DTYPE_BF16, 80, 4, 1, 4096) == -1
