@@ -444,20 +444,28 @@ int select_base(const fl::FwdArgs& a) {
 // masks, us per call; fp16 figures, bf16 within 3% of them):
 //  - at most one 32-row block per CU, square causal 1.5 (their lengths
 //    differ; 1.25-1.5 non-causal lose 3-11%): the 32-row groups (figures in
-//    fa2_rows32.hip; B2 H8 N640 causal 7.35 against 7.9), but for 257-512 keys
-//    with at most 5/8 of a block per CU the key quarters, whose waves hold
-//    both their tiles at once (B1 H8 N384 5.05 against 5.35, B1 H16 N300 5.28
-//    against 5.56; at 256 blocks B2 H8 N512 7.3 against 5.6).  Q rows must lie
+//    fa2_rows32.hip; B2 H8 N640 causal 7.35 against 7.9).  Q rows must lie
 //    within the buffer offsets of a block (2^24 elements apart);
+//  - 257-512 keys with at most two blocks per CU: the key quarters, whose
+//    waves hold both their tiles at once, up to 5/8 of a block per CU (B1 H8
+//    N384 5.05 against 5.35, B1 H16 N300 5.28 against 5.56) and for at most 32
+//    query rows per head up to one (B16 H16 30 x 300 6.9 against 7.8); else
+//    the 32-row groups, two per CU (new inputs each call: B2 H8 N512 6.25
+//    against 7.1, B2 H16 N512 8.2 against 10.8, B30 H10 one row over 400 keys
+//    10.6 against 15.4).  The 64-row split was faster still (B2 H16 N512 7.1
+//    in graphs against 7.8), but only its ranges' first 32 keys set the
+//    stabiliser: 7% more error against 64 bits, 2.88e-4 against 2.70e-4 for
+//    the quarters and 2.66e-4 for the 32-row groups;
 //  - up to 256 keys beyond that: the 64-row split while it fits one round and
 //    has four tiles (B4 H16 N256 5.95 against 6.3; at N192 5.9 against 5.7),
 //    the streaming groups from 1024 units of 256 rows and 128 keys (B32 H32
-//    N128 16.1 against 16.9, causal N256 32.7 against 39.2) or 512 causal ones
-//    past 192 keys (B16 H32 N256 17.4 against 19.4), else the 4-wave groups
-//    (B8 H16 N256 7.7 against 9.0 streaming, B16 H32 N96 8.6 against 10.0);
+//    N128 16.1 against 16.9, causal N256 32.7 against 39.2), 512 causal ones
+//    past 192 keys (B16 H32 N256 17.4 against 19.4), or non-causal up to 192
+//    keys (the 4-wave groups were faster, B16 H32 N96 8.6 against 10.0, but
+//    0.2-0.8% further from 64 bits); else the 4-wave groups (B8 H16 N256 7.7
+//    against 9.0 streaming);
 //  - at most one 64-row group per CU, causal from 1280 keys 1.5: the 64-row
-//    split (B2 H16 N512 7.1 against 11.3 on the key quarters' 8-wave groups,
-//    B2 H8 N1280 causal 12.1 against 14.2, B1 H8 N3000 causal 20.1 against
+//    split (B2 H8 N1280 causal 12.1 against 14.2, B1 H8 N3000 causal 20.1 against
 //    22.0; at N640-768 causal with 1.25-1.5 it lost 10-15%);
 //  - square causal from 1792 keys with at most one pair of 64-row blocks per
 //    CU: the 64-row pairs (B2 H8 N1999 17.9 against 18.4 for the 128-row split;
@@ -474,15 +482,17 @@ int select_d64_fast(const fl::FwdArgs& a) {
   auto wgs = [&](int64_t br) { return (a.seq + br - 1) / br * (int64_t)a.batch_heads; };
   const bool square = a.causal && a.seq == a.seq_k;
   const bool few = a.seq <= 32 && a.batch_heads >= cus;  // decode over many heads
-  if (!few && a.q_sr <= (1 << 24) && wgs(32) <= (square ? cus + cus / 2 : cus)) {
-    if (a.seq_k > 256 && fl::quarter_config_fits(a) && 8 * wgs(32) <= 5 * cus)
-      return fl::kQuarterConfig;
-    return fl::kRows32Config;
+  const bool rows32 = a.q_sr <= (1 << 24);
+  const bool quarter = a.seq_k > 256 && fl::quarter_config_fits(a) && wgs(32) <= 2 * cus;
+  if (quarter) {
+    const bool keep = 8 * wgs(32) <= 5 * cus || (a.seq <= 32 && wgs(32) <= cus);
+    return !rows32 || keep ? fl::kQuarterConfig : fl::kRows32Config;
   }
+  if (!few && rows32 && wgs(32) <= (square ? cus + cus / 2 : cus)) return fl::kRows32Config;
   if (a.seq_k <= 256) {
     if (a.seq_k > 192 && wgs(64) <= cus) return fl::kCfgSplit2W2;
     if (fl::stream_config_fits(a) &&
-        ((a.seq_k >= 128 && wgs(256) >= 4 * cus) ||
+        ((!a.causal && a.seq_k <= 192) || (a.seq_k >= 128 && wgs(256) >= 4 * cus) ||
          (a.causal && a.seq_k > 192 && wgs(256) >= 2 * cus)))
       return fl::kStreamConfig;
     return fl::kSlotW4Config;

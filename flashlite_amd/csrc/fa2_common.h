@@ -725,18 +725,22 @@ struct Rows {
   __device__ __forceinline__ void softmax_checked(float16_t (&s)[2], V8 (&pn)[2][2]) {
     float sum = exponentiate(s, pn);
     if (__builtin_amdgcn_ballot_w64(!(sum <= kSumLimit)) != 0) {
-      const float d = fmaxf(tile_max(s), 0.0f);
-      const float alpha = __builtin_amdgcn_exp2f(-(SCALED ? cr : 1.0f) * d);
-      l *= alpha;
-#pragma unroll
-      for (int db = 0; db < 2; ++db)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o[db][r] *= alpha;
-      sub(s, d);
-      set_m(m + d);
+      raise_m(s);
       sum = exponentiate(s, pn);
     }
     l += sum;
+  }
+  // m moves up to the row max of tile s, if that is larger, with O, l and s.
+  __device__ __forceinline__ void raise_m(float16_t (&s)[2]) {
+    const float d = fmaxf(tile_max(s), 0.0f);
+    const float alpha = __builtin_amdgcn_exp2f(-(SCALED ? cr : 1.0f) * d);
+    l *= alpha;
+#pragma unroll
+    for (int db = 0; db < 2; ++db)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[db][r] *= alpha;
+    sub(s, d);
+    set_m(m + d);
   }
   // Row max of a tile (both halves of the row).
   __device__ __forceinline__ float tile_max(const float16_t (&s)[2]) const {

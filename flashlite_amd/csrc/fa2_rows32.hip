@@ -25,7 +25,7 @@ namespace {
 // tiles, two groups per CU; NW = 8, one group per CU, serves long walks.
 // Against the configurations the dispatcher took before (fp16 and bf16 alike
 // at head dim 64, us per call): B1 H1 N128 5.05 -> 4.35, B2 H8 N256 7.2 ->
-// 4.8, B2 H8 N512 7.3 -> 5.6, B1 H8 N1024 8.9 -> 6.9, B1 H2 N4096 causal 21.4
+// 4.8, B2 H8 N512 7.0 -> 5.8, B1 H8 N1024 8.9 -> 6.9, B1 H2 N4096 causal 21.4
 // -> 14.2 (NW = 8; 15.9 with 4), B1 H1 N8192 36.8 -> 29.4; head dim 128: B2
 // H8 N512 8.55 -> 6.97, B1 H2 N4096 30.9 -> 25.6.  Two tiles in flight per
 // wave (128 KiB, one group per CU) measured 0-10% slower than one.
@@ -46,9 +46,9 @@ struct TileRows<128, T, CAUSAL> : Rows128<CAUSAL, T> {
   __device__ __forceinline__ void scores(const uint8_t* kt, Scores& s) const {
     this->gemm1(kt, s.s);
   }
-  __device__ __forceinline__ void softmax(int t, bool first, Scores& s, Probs& p) {
+  __device__ __forceinline__ void softmax(int t, int i, Scores& s, Probs& p) {
     this->mask(t, s.s);
-    if (first) this->first_tile(s.s);
+    if (i == 0) this->first_tile(s.s);
     this->softmax_checked(s.s, p.p);
   }
   __device__ __forceinline__ void output(const uint8_t* vt, const Probs& p) {
@@ -77,9 +77,16 @@ struct TileRows<64, T, CAUSAL> : Rows<CAUSAL, true, T> {
     this->read_k(kt, ka);
     this->gemm1(ka, s.s);
   }
-  __device__ __forceinline__ void softmax(int t, bool first, Scores& s, Probs& p) {
+  // The stabiliser is the exact row max over the first two tiles, so the
+  // largest p of a walk of up to 512 keys is 1 and rounds to itself: a row's
+  // error is mostly that of its few largest p (B2 H8 N512 against 64 bits
+  // 2.78e-4 with the first tile's max, 2.66e-4 so; 0.3 us a call).
+  __device__ __forceinline__ void softmax(int t, int i, Scores& s, Probs& p) {
     this->mask(t, s.s);
-    if (first) this->first_tile(s.s);
+    if (i == 0)
+      this->first_tile(s.s);
+    else if (i == 1)
+      this->raise_m(s.s);
     this->softmax_checked(s.s, p.p);
   }
   __device__ __forceinline__ void output(const uint8_t* vt, const Probs& p) {
@@ -161,7 +168,7 @@ fa2_fwd_rows32_kernel(const T* Q, const T* __restrict__ K, const T* __restrict__
     rows.scores(buf[w][0], s);
     asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");  // its operands are in registers
     fetch_k(i + 1);
-    rows.softmax(mine0 + NW * i, i == 0, s, p);
+    rows.softmax(mine0 + NW * i, i, s, p);
     asm volatile("s_waitcnt vmcnt(8)" : : : "memory");  // V(i)
     rows.output(buf[w][1], p);
     asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");

@@ -78,3 +78,13 @@ def test_lse_sums_stay_fp32(cuda, kind, h, nq, nk):
     assert error_stats(lse, attention_lse(q, k, 0.125, False))[0] <= 1e-5
     out, _ = run_wide(kind, q, k, v, 0.125, False, cuda)
     assert_close_oracle(out, None, None, None, 0.125, False, max_abs=mx, mean_abs=mean, ref=ref)
+
+
+@pytest.mark.parametrize("kind", ["fp16", "bf16"])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("h,nq,nk", [(12, 700, 257), (16, 1024, 512), (264, 20, 300)])
+def test_two_groups_per_cu(cuda, kind, causal, h, nq, nk):
+    """257-512 keys over one to two 32-row blocks per CU: two tiles per wave,
+    the second of which raises the stabiliser in about half the rows."""
+    check(kind, 64, nq, nk, 0.125, causal, cuda, h=h)
+    check(kind, 64, nq, nk, 1.0, causal, cuda, scale=1.5, h=h)
