@@ -217,8 +217,10 @@ fa2_fwd_kernel(const _Float16* Q, const _Float16* __restrict__ K,
 // N_q 4 N_k 8192, 16 chunks: 12.2 -> 11.5).  Beyond, each
 // batch of 8 chunks issues its O loads before the first multiply; up-front
 // batches there measured up to 15% slower (128 and more chunks).  A chunk with
-// no visible key stored m = -inf and l = 0: weight 0, skipped by a select, not
-// a branch.
+// no visible key stored m = -inf and l = 0: weight kSkip, passed over by a
+// select, not a branch.  A NaN score makes its chunk's l NaN (whatever m says),
+// and with it the row's sum and output, as in one pass; a weight that
+// underflows to 0 still multiplies its chunk, so a NaN or infinity in V shows.
 __device__ __forceinline__ float wave_max64(float x) {
 #pragma unroll
   for (int m = 32; m >= 1; m >>= 1) x = fmaxf(x, __shfl_xor(x, m, 64));
@@ -245,11 +247,16 @@ splitkv_combine_kernel(T* O, const Geom geom) {
   const float* p0 = geom.part + (long long)row_id * kPart;
   const int ns = geom.nsplit;
   float acc[kCols] = {}, lpart = 0.0f, mx;
-  // Chunk s0 + j's weight, from lane j of w; a weight of 0 skips the chunk.
+  constexpr float kSkip = -1.0f;  // weights are >= 0
+  // Chunk s0 + j's weight, from lane j of w.
   auto fold = [&](float w, int j, const float (&x)[kCols]) __attribute__((always_inline)) {
     const float wj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), j));
 #pragma unroll
-    for (int c = 0; c < kCols; ++c) acc[c] += wj == 0.0f ? 0.0f : wj * x[c];
+    for (int c = 0; c < kCols; ++c) acc[c] += wj == kSkip ? 0.0f : wj * x[c];
+  };
+  // The weight of a chunk with stabiliser m, given the row's largest.
+  auto weight = [&](float m) __attribute__((always_inline)) {
+    return m == ninf() ? kSkip : __builtin_amdgcn_exp2f(m - mx);
   };
   auto load = [&](int s, float (&x)[kCols]) __attribute__((always_inline)) {
 #pragma unroll
@@ -261,7 +268,7 @@ splitkv_combine_kernel(T* O, const Geom geom) {
       m = p0[lane * split_stride + D];
       l = p0[lane * split_stride + D + 1];
     }
-    // (past the last chunk: its values again, weight 0)
+    // (past the last chunk: its values again, passed over)
     float o[kUpFront][kBatch][kCols];
 #pragma unroll
     for (int i = 0; i < kUpFront; ++i)
@@ -270,8 +277,8 @@ splitkv_combine_kernel(T* O, const Geom geom) {
         for (int u = 0; u < kBatch; ++u) load(min(i * kBatch + u, ns - 1), o[i][u]);
       }
     mx = wave_max64(m);
-    const float w = m == ninf() ? 0.0f : __builtin_amdgcn_exp2f(m - mx);
-    lpart = w * l;
+    const float w = weight(m);
+    lpart = fmaxf(w, 0.0f) * l;
 #pragma unroll
     for (int i = 0; i < kUpFront; ++i)
       if (i == 0 || ns > i * kBatch) {
@@ -283,11 +290,10 @@ splitkv_combine_kernel(T* O, const Geom geom) {
     for (int s = lane; s < ns; s += 64) mx = fmaxf(mx, p0[s * split_stride + D]);
     mx = wave_max64(mx);
     for (int s0 = 0; s0 < ns; s0 += 64) {
-      float w = 0.0f;
+      float w = kSkip;
       if (s0 + lane < ns) {
-        const float m = p0[(s0 + lane) * split_stride + D];
-        w = m == ninf() ? 0.0f : __builtin_amdgcn_exp2f(m - mx);
-        lpart += w * p0[(s0 + lane) * split_stride + D + 1];
+        w = weight(p0[(s0 + lane) * split_stride + D]);
+        lpart += fmaxf(w, 0.0f) * p0[(s0 + lane) * split_stride + D + 1];
       }
       const int cnt = min(64, ns - s0);
       int j = 0;
@@ -310,7 +316,7 @@ splitkv_combine_kernel(T* O, const Geom geom) {
   T* orow = O + (b * geom.o_sb + h * geom.o_sh) + (long long)row * geom.o_sr;
 #pragma unroll
   for (int c = 0; c < kCols; ++c)
-    orow[lane + 64 * c] = (T)(lsum > 0.0f ? acc[c] / lsum : 0.0f);
+    orow[lane + 64 * c] = (T)(lsum == 0.0f ? 0.0f : acc[c] / lsum);
   if (geom.lse != nullptr && lane == 0)
     geom.lse[row_id] =
         lsum > 0.0f ? 0.693147180559945309f * (mx + __builtin_amdgcn_logf(lsum)) : ninf();
