@@ -444,8 +444,7 @@ int select_base(const fl::FwdArgs& a) {
 // masks, us per call; fp16 figures, bf16 within 3% of them):
 //  - at most one 32-row block per CU, square causal 1.5 (their lengths
 //    differ; 1.25-1.5 non-causal lose 3-11%): the 32-row groups (figures in
-//    fa2_rows32.hip; B2 H8 N640 causal 7.35 against 7.9).  Q rows must lie
-//    within the buffer offsets of a block (2^24 elements apart);
+//    fa2_rows32.hip; B2 H8 N640 causal 7.35 against 7.9);
 //  - 257-512 keys with at most two blocks per CU: the key quarters, whose
 //    waves hold both their tiles at once, up to 5/8 of a block per CU (B1 H8
 //    N384 5.05 against 5.35, B1 H16 N300 5.28 against 5.56) and for at most 32
@@ -482,13 +481,12 @@ int select_d64_fast(const fl::FwdArgs& a) {
   auto wgs = [&](int64_t br) { return (a.seq + br - 1) / br * (int64_t)a.batch_heads; };
   const bool square = a.causal && a.seq == a.seq_k;
   const bool few = a.seq <= 32 && a.batch_heads >= cus;  // decode over many heads
-  const bool rows32 = a.q_sr <= (1 << 24);
   const bool quarter = a.seq_k > 256 && fl::quarter_config_fits(a) && wgs(32) <= 2 * cus;
   if (quarter) {
     const bool keep = 8 * wgs(32) <= 5 * cus || (a.seq <= 32 && wgs(32) <= cus);
-    return !rows32 || keep ? fl::kQuarterConfig : fl::kRows32Config;
+    return keep ? fl::kQuarterConfig : fl::kRows32Config;
   }
-  if (!few && rows32 && wgs(32) <= (square ? cus + cus / 2 : cus)) return fl::kRows32Config;
+  if (!few && wgs(32) <= (square ? cus + cus / 2 : cus)) return fl::kRows32Config;
   if (a.seq_k <= 256) {
     if (a.seq_k > 192 && wgs(64) <= cus) return fl::kCfgSplit2W2;
     if (fl::stream_config_fits(a) &&
@@ -565,7 +563,7 @@ WsPlan plan_ws(const fl::FwdArgs& a) {
   const int64_t tiles = (a.seq_k + keys - 1) / keys;
   const int64_t row = a.head_dim == 64 ? kPartFloats : kPartFloats128;
   if (a.seq > 32 || 2 * heads >= cus) return p;
-  // the 32-row groups' buffer offsets within a Q block (fetch_q_block)
+  // Q rows past the reach of a block's DMA (fetch_q_block): one pass
   if (a.head_dim == 64 && a.q_sr > (1 << 24)) return p;
   int64_t n, least;
   if (8 * heads <= cus) {

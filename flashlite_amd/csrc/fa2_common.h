@@ -389,20 +389,35 @@ __device__ __forceinline__ void fetch_seg(const i32x4_t& rs, const uint8_t* slot
   asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" : : "v"(voff), "s"(rs), "{m0}"(lds_base));
 }
 
-// DMA of the 32 query rows [q, q + 32) of a head (rows >= N_q read as
-// zeros) into `qblk`, laid out as the first half of a K tile (Rows::
-// set_q_lds reads it): 4 fetches of 1 KiB, counted by vmcnt, or with kParts
-// waves sharing the block, the 4 / kParts of them of part `part`.
+// The 32 query rows [q, q + 32) of a head (rows >= N_q read as zeros) into
+// `qblk`, laid out as the first half of a K tile (Rows::set_q_lds reads it):
+// 4 fetches of 1 KiB by DMA, counted by vmcnt, or with kParts waves sharing
+// the block, the 4 / kParts of them of part `part`.  Rows further apart than
+// 32-bit offsets reach over a block go through registers; the LDS writes are
+// then what the caller's lgkmcnt wait before its barrier completes.
+constexpr int kDmaQRowStride = 1 << 24;  // 31 rows of it: 2^30 bytes
+
 template <int kParts = 1, class T>
 __device__ __forceinline__ void fetch_q_block(const T* Qh, int q_sr, int q, int seq,
                                               uint8_t* qblk, int lane, int part = 0) {
   static_assert(kParts == 1 || kParts == 2 || kParts == 4, "Q block parts");
   constexpr int kSegs = 4 / kParts;
   const int rows = min(32, seq - q);
-  const i32x4_t rq = buffer_rsrc(Qh + (long long)(rows > 0 ? q : 0) * q_sr,
-                                 rows > 0 ? (rows - 1) * (2 * q_sr) + kRowBytes : 0);
-  const FetchOff<kSegs> fq = fetch_offsets<kSegs, false>(part, lane, 2 * q_sr);
-  fetch_tile_z<kSegs>(rq, qblk, 0, 1, part, fq);
+  if (q_sr <= kDmaQRowStride) {
+    const i32x4_t rq = buffer_rsrc(Qh + (long long)(rows > 0 ? q : 0) * q_sr,
+                                   rows > 0 ? (rows - 1) * (2 * q_sr) + kRowBytes : 0);
+    const FetchOff<kSegs> fq = fetch_offsets<kSegs, false>(part, lane, 2 * q_sr);
+    fetch_tile_z<kSegs>(rq, qblk, 0, 1, part, fq);
+  } else {
+#pragma unroll 1
+    for (int i = 0; i < kSegs; ++i) {
+      const int row = 8 * (part * kSegs + i) + (lane >> 3), chunk = lane & 7;
+      u32x4_t x = {0, 0, 0, 0};
+      if (row < rows)
+        x = *reinterpret_cast<const u32x4_t*>(Qh + (long long)(q + row) * q_sr + 8 * chunk);
+      *reinterpret_cast<u32x4_t*>(qblk + row * kRowBytes + 16 * (chunk ^ k_swz(row))) = x;
+    }
+  }
 }
 
 template <int kSegs>

@@ -294,7 +294,7 @@ __device__ __forceinline__ void fetch_q_block128(const T* Qh, int q_sr, int q, i
                                                  uint8_t* qblk, int lane, int part) {
   constexpr int kSegs = 8 / kParts;
   const int rows = min(32, seq - q);
-  if (q_sr <= (1 << 24)) {
+  if (q_sr <= kDmaQRowStride) {
     const i32x4_t rq = buffer_rsrc(Qh + (long long)(rows > 0 ? q : 0) * q_sr,
                                    rows > 0 ? (rows - 1) * (2 * q_sr) + kRowBytes2 : 0);
     const FetchOff<kSegs> fq = fetch_offsets128<kSegs, false>(part, lane, 2 * q_sr);

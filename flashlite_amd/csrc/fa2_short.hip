@@ -117,13 +117,7 @@ fa2_fwd_quarter_kernel(const T* Q, const T* __restrict__ K, const T* __restrict_
   // K of its first tile has landed.  Tiles past the quarter land as zeros
   // with no traffic.
   const int qr = q0 + 32 * rb;  // this wave's rows
-  {
-    const int qrows = min(32, seq - qr);
-    const i32x4_t rq = buffer_rsrc(hp.q + (long long)(qrows > 0 ? qr : 0) * geom.q_sr,
-                                   qrows > 0 ? (qrows - 1) * (2 * geom.q_sr) + kRowBytes : 0);
-    const FetchOff<1> fq = fetch_offsets<1, false>(kq, lane, 2 * geom.q_sr);
-    fetch_tile_z<1>(rq, qblk, 0, 1, kq, fq);
-  }
+  fetch_q_block<NW>(hp.q, geom.q_sr, qr, seq, qblk, lane, kq);
   i32x4_t rk, rv;
   kv_rsrc_rows(geom, bh, K, V, t1 * kBc, rk, rv);
   const bool any = t0 < t1;
