@@ -455,14 +455,9 @@ int select_base(const fl::FwdArgs& a) {
 //    in graphs against 7.8), but only its ranges' first 32 keys set the
 //    stabiliser: 7% more error against 64 bits, 2.88e-4 against 2.70e-4 for
 //    the quarters and 2.66e-4 for the 32-row groups;
-//  - up to 256 keys beyond that: the 64-row split while it fits one round and
-//    has four tiles (B4 H16 N256 5.95 against 6.3; at N192 5.9 against 5.7),
-//    the streaming groups from 1024 units of 256 rows and 128 keys (B32 H32
-//    N128 16.1 against 16.9, causal N256 32.7 against 39.2), 512 causal ones
-//    past 192 keys (B16 H32 N256 17.4 against 19.4), or non-causal up to 192
-//    keys (the 4-wave groups were faster, B16 H32 N96 8.6 against 10.0, but
-//    0.2-0.8% further from 64 bits); else the 4-wave groups (B8 H16 N256 7.7
-//    against 9.0 streaming);
+//  - up to 256 keys beyond that: the streaming groups.  The 64-row split (B4
+//    H16 N256 5.95 against 6.3) and the 4-wave groups (B8 H16 N256 7.7 against
+//    9.0) are faster, but sum the p that are rounded to 16 bits;
 //  - at most one 64-row group per CU, causal from 1280 keys 1.5: the 64-row
 //    split (B2 H8 N1280 causal 12.1 against 14.2, B1 H8 N3000 causal 20.1 against
 //    22.0; at N640-768 causal with 1.25-1.5 it lost 10-15%);
@@ -476,25 +471,19 @@ int select_base(const fl::FwdArgs& a) {
 //    only from 4096 keys or where their last round is nearly full (B2 H16
 //    N3000, 1.5 rounds, 91.3 against 79.9 on the 4-wave groups).
 // Beyond these, the base rule.
-int select_d64_fast(const fl::FwdArgs& a) {
+int select_d64(const fl::FwdArgs& a) {
   const int64_t cus = fl::device_cus();
   auto wgs = [&](int64_t br) { return (a.seq + br - 1) / br * (int64_t)a.batch_heads; };
   const bool square = a.causal && a.seq == a.seq_k;
   const bool few = a.seq <= 32 && a.batch_heads >= cus;  // decode over many heads
-  const bool quarter = a.seq_k > 256 && fl::quarter_config_fits(a) && wgs(32) <= 2 * cus;
+  const bool quarter =
+      !fl::stream_config_fits(a) && fl::quarter_config_fits(a) && wgs(32) <= 2 * cus;
   if (quarter) {
     const bool keep = 8 * wgs(32) <= 5 * cus || (a.seq <= 32 && wgs(32) <= cus);
     return keep ? fl::kQuarterConfig : fl::kRows32Config;
   }
   if (!few && wgs(32) <= (square ? cus + cus / 2 : cus)) return fl::kRows32Config;
-  if (a.seq_k <= 256) {
-    if (a.seq_k > 192 && wgs(64) <= cus) return fl::kCfgSplit2W2;
-    if (fl::stream_config_fits(a) &&
-        ((!a.causal && a.seq_k <= 192) || (a.seq_k >= 128 && wgs(256) >= 4 * cus) ||
-         (a.causal && a.seq_k > 192 && wgs(256) >= 2 * cus)))
-      return fl::kStreamConfig;
-    return fl::kSlotW4Config;
-  }
+  if (fl::stream_config_fits(a)) return fl::kStreamConfig;
   if (few) return fl::kSlotW4Config;
   if (wgs(64) <= (a.causal && a.seq_k >= 1280 ? cus + cus / 2 : cus)) return fl::kCfgSplit2W2;
   const int64_t pairs64 = (((int64_t)a.seq + 63) / 64 + 1) / 2 * a.batch_heads;
@@ -506,22 +495,6 @@ int select_d64_fast(const fl::FwdArgs& a) {
       10 * g < 9 * rounds * cus)
     return fl::kSlotW4Config;
   return c;
-}
-
-// The log-sum-exp keeps its precision: the slot schedules sum the rounded p
-// (about 1e-5 of ln l), the other kernels the fp32 p, so a call that asks for
-// it and that the base rule gives one of those does not move to a slot
-// schedule.
-bool rounded_sums(int cfg) {
-  return cfg == fl::kCfgSplit2 || cfg == fl::kSlotW8Config || cfg == fl::kSlotW4Config ||
-         cfg == fl::kCfgSplit2W2 || cfg == fl::kCfgPair || cfg == fl::kCfgPairW2;
-}
-
-int select_d64(const fl::FwdArgs& a) {
-  const int c = select_d64_fast(a);
-  if (a.lse == nullptr || !rounded_sums(c)) return c;
-  const int base = select_base(a);
-  return rounded_sums(base) ? c : base;
 }
 
 int select_any(const fl::FwdArgs& a) {

@@ -7,6 +7,7 @@ keys).  Tolerances: gpu_util (against the fp32 oracle).
 import numpy as np
 import pytest
 
+import flashlite_amd as fl
 from gpu_util import (LSE_MAX_ABS, LSE_MEAN_ABS, assert_close_oracle, run_wide, wide_inputs,
                       wide_tol)
 from oracle import attention_fp32, attention_lse, error_stats
@@ -78,6 +79,25 @@ def test_lse_sums_stay_fp32(cuda, kind, h, nq, nk):
     assert error_stats(lse, attention_lse(q, k, 0.125, False))[0] <= 1e-5
     out, _ = run_wide(kind, q, k, v, 0.125, False, cuda)
     assert_close_oracle(out, None, None, None, 0.125, False, max_abs=mx, mean_abs=mean, ref=ref)
+
+
+@pytest.mark.parametrize("kind", ["fp16", "bf16"])
+@pytest.mark.parametrize("h,nq,nk,causal", [
+    (40, 193, 193, False), (64, 256, 256, True), (96, 129, 129, True), (128, 200, 200, False),
+    (160, 192, 192, True), (300, 100, 97, False), (300, 5, 256, True), (600, 130, 130, True)])
+def test_one_kernel_with_and_without_lse(cuda, kind, h, nq, nk, causal):
+    """The output does not depend on whether the log-sum-exp is asked for: up
+    to 256 keys both calls sum the fp32 p (test_lse_sums_stay_fp32), never
+    p rounded to 16 bits."""
+    import torch
+
+    g = torch.Generator(device="cpu")
+    g.manual_seed(h + nq + nk)
+    dt = torch.bfloat16 if kind == "bf16" else torch.float16
+    q = torch.randn((1, h, nq, 64), generator=g).to(cuda).to(dt)
+    k, v = (torch.randn((1, h, nk, 64), generator=g).to(cuda).to(dt) for _ in range(2))
+    out, _ = fl.forward_flash2_ex(q, k, v, 0.125, causal, return_lse=True)
+    assert torch.equal(out, fl.forward_flash2_ex(q, k, v, 0.125, causal))
 
 
 @pytest.mark.parametrize("kind", ["fp16", "bf16"])
