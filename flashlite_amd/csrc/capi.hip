@@ -721,6 +721,7 @@ int fl_attn_fwd_ws(const fl_attn_params_ex* p, int32_t dtype, void* workspace,
 int64_t fl_attn_splitkv_workspace_bytes(const fl_attn_params_ex* p, int32_t num_splits) {
   fl::FwdArgs a;
   if (check_ex(p, &a, "fl_attn_splitkv_workspace_bytes") != FL_OK) return -1;
+  if (empty_problem(a)) return 0;
   const KvPlan plan = plan_kvsplit(a, num_splits);
   return plan.nsplit == 0 ? 0 : plan.bytes;
 }
@@ -728,6 +729,7 @@ int64_t fl_attn_splitkv_workspace_bytes(const fl_attn_params_ex* p, int32_t num_
 int64_t fl_attn_splitkv_noalloc_bytes(const fl_attn_params_ex* p, int32_t num_splits) {
   fl::FwdArgs a;
   if (check_ex(p, &a, "fl_attn_splitkv_noalloc_bytes") != FL_OK) return -1;
+  if (empty_problem(a)) return 0;
   const KvPlan plan = plan_kvsplit_capped(a, num_splits, FL_ATTN_SCRATCH_BYTES);
   return plan.nsplit == 0 ? 0 : plan.bytes;
 }

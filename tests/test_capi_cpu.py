@@ -407,3 +407,14 @@ def test_config_id_lookup():
     assert capi.load().fl_attn_config_id(None) == -1
     with pytest.raises(KeyError):
         capi.config_id("no_such_config")
+
+
+@pytest.mark.parametrize("batch,heads,nq", [(0, 4, 1), (2, 0, 1), (2, 4, 0)])
+def test_size_queries_of_empty_problems(batch, heads, nq):
+    # no row to write: no workspace, for the library's choice and a given count
+    p = _ex_shape(batch, heads, nq, 4096)
+    for splits in (0, 8):
+        assert capi.splitkv_workspace_bytes(p, splits) == 0
+        assert capi.splitkv_noalloc_bytes(p, splits) == 0
+    assert capi.workspace_bytes(p, capi.DTYPE_F16) == 0
+    assert capi.workspace_bytes(p, capi.DTYPE_BF16) == 0
