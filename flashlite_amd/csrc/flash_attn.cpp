@@ -61,18 +61,6 @@ bool usable_workspace(const torch::Tensor& ws, const torch::Tensor& q) {
          reinterpret_cast<uintptr_t>(ws.data_ptr()) % 16 == 0;
 }
 
-// A wide call with `out` given allocated nothing, so it could be captured by
-// means the caching allocator does not see; under capture it still allocates
-// nothing.
-bool capturing(void* stream) {
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(static_cast<hipStream_t>(stream), &st) != hipSuccess) {
-    (void)hipGetLastError();  // not the next launch's error
-    return false;
-  }
-  return st != hipStreamCaptureStatusNone;
-}
-
 }  // namespace
 
 torch::Tensor flash_attn_forward_naive(torch::Tensor q, torch::Tensor k, torch::Tensor v,
@@ -161,8 +149,12 @@ torch::Tensor flash_attn_forward_flash2(torch::Tensor q, torch::Tensor k, torch:
 // num_splits: 0 = the library's choice, 1 = one pass, n > 1 = n key chunks
 // (fp16 at head_dim 64).
 // A split-KV call needs a workspace: `workspace` (any device tensor of
-// enough bytes, reused across calls for an allocation-free loop) or else
-// one from the caching allocator.
+// enough bytes, reused across calls for an allocation-free loop; calls that
+// may overlap on the GPU must not share one) or else one from the caching
+// allocator.  bf16 and head_dim 128 (`wide`) take one from the allocator only
+// where the call allocates its output or log-sum-exp anyway; with both given
+// and no `workspace` they run one pass and allocate nothing, eagerly and under
+// capture alike.
 py::object flash_attn_forward_flash2_ex(torch::Tensor q, torch::Tensor k, torch::Tensor v,
                                         double sm_scale, bool is_causal,
                                         std::optional<torch::Tensor> out, bool return_lse,
@@ -190,7 +182,8 @@ py::object flash_attn_forward_flash2_ex(torch::Tensor q, torch::Tensor k, torch:
   check_same_device(q, k, v);
 
   torch::Tensor out_tensor;
-  if (out.has_value() && out.value().defined()) {
+  const bool out_given = out.has_value() && out.value().defined();
+  if (out_given) {
     out_tensor = out.value();
     TORCH_CHECK(out_tensor.is_cuda() && out_tensor.stride(3) == 1,
                 "out tensor must be a CUDA tensor with a unit-stride head dimension");
@@ -229,6 +222,7 @@ py::object flash_attn_forward_flash2_ex(torch::Tensor q, torch::Tensor k, torch:
   const bool wide = bf16 || head_dim != 64;
   TORCH_CHECK(!wide || num_splits <= 1,
               "split-KV (num_splits > 1) needs fp16 tensors with head_dim 64");
+  const bool allocates = !out_given || (return_lse && !lse_given);
   const int32_t dtype = bf16 ? FL_DTYPE_BF16 : FL_DTYPE_F16;
   const int64_t ws_bytes = num_splits == 1 ? 0
                            : num_splits == 0
@@ -251,11 +245,11 @@ py::object flash_attn_forward_flash2_ex(torch::Tensor q, torch::Tensor k, torch:
                   "workspace must be a contiguous tensor on q's device");
       buf = ws.data_ptr();
       have = ws.nbytes();
-    } else if (!wide || !capturing(current_stream(q))) {
+    } else if (!wide || allocates) {
       ws = torch::empty({(ws_bytes + 3) / 4}, q.options().dtype(torch::kFloat32));
       buf = ws.data_ptr();
       have = ws.nbytes();
-    }  // a wide call under capture without a workspace: one pass, nothing allocated
+    }  // else one pass
     rc = num_splits == 0 ? fl_attn_fwd_ws(&p, dtype, buf, (int64_t)have, current_stream(q))
                          : fl_attn_fwd_f16_splitkv(&p, (int32_t)num_splits, buf, (int64_t)have,
                                                    current_stream(q));
@@ -280,7 +274,10 @@ PYBIND11_MODULE(flash_attn_wmma, m) {
 
   m.def("forward_flash2_ex", &flash_attn::flash_attn_forward_flash2_ex,
         "FlashAttention-2 forward on strided [B, H, N, D] views (fp16 or bf16, D 64 or 128), "
-        "N_k != N_q (bottom-right causal), optional log-sum-exp",
+        "N_k != N_q (bottom-right causal), optional log-sum-exp.  Few query rows over many keys "
+        "run as key chunks through `workspace` (splitkv_workspace_bytes bytes on q's device); "
+        "calls that may overlap on the GPU must not share one.  Without it bf16 and head_dim 128 "
+        "calls that are given their outputs run one pass and allocate nothing",
         py::arg("q"), py::arg("k"), py::arg("v"), py::arg("sm_scale") = 0.0,
         py::arg("is_causal") = false, py::arg("out") = py::none(), py::arg("return_lse") = false,
         py::arg("num_splits") = 0, py::arg("workspace") = py::none(), py::arg("lse") = py::none());

@@ -95,6 +95,28 @@ def test_binding_and_graph(cuda, kind, d):
             torch.empty(1 << 20, device=cuda).fill_(1.0)
 
 
+@pytest.mark.parametrize("kind,d", WIDE)
+def test_given_outputs_allocate_nothing(cuda, kind, d):
+    """Without a workspace (or with one too small) a call that is given its
+    outputs makes no allocation: one pass, the same bits as under capture."""
+    import torch
+
+    q, k, v = tensors(kind, wide_inputs(kind, 2, 4, 1, 3000, d, seed=5), cuda)
+    one, one_lse = fl.forward_flash2_ex(q, k, v, 0.125, return_lse=True, num_splits=1)
+    out, lse = torch.empty_like(one), torch.empty_like(one_lse)
+    small = torch.empty(16, dtype=torch.float32, device=cuda)
+    count = lambda: torch.cuda.memory_stats(cuda)["allocation.all.allocated"]  # noqa: E731
+    for w in (None, small):
+        out.fill_(float("nan"))
+        torch.cuda.synchronize(cuda)
+        n = count()
+        fl.forward_flash2_ex(q, k, v, 0.125, out=out, workspace=w)
+        fl.forward_flash2_ex(q, k, v, 0.125, out=out, return_lse=True, lse=lse, workspace=w)
+        assert count() == n
+        torch.cuda.synchronize(cuda)
+        assert torch.equal(out, one) and torch.equal(lse, one_lse)
+
+
 def test_refused_chunk_counts(cuda):
     q, k, v = tensors("bf16", wide_inputs("bf16", 1, 2, 1, 3000, 64, seed=4), cuda)
     with pytest.raises(RuntimeError, match="num_splits > 1"):
