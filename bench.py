@@ -254,8 +254,8 @@ def main():
         torch.cuda.synchronize()
         gpu_out[causal] = out.float().cpu().numpy().astype(np.float64)
 
-    p = capi.tensor_params(q, k, v, out, w.sm_scale, False)
-    cfg = capi.select_config(p)
+    tile_config = capi.launch_name(capi.tensor_params_ex(q, k, v, out, w.sm_scale, False),
+                                   capi.DTYPE_F16)
     nc, ca = results[False], results[True]
     value = nc["flops"] / (nc["wall_ms"] * 1e-3) / 1e12
     achieved = nc["flops"] / (nc["kern_ms"] * 1e-3) / 1e12
@@ -284,7 +284,7 @@ def main():
                 % w.seed,
         "config": {"workload": HEADLINE, "batch": w.batch, "heads": w.heads, "seq_len": w.seq,
                    "head_dim": w.head_dim, "causal": False, "sm_scale": w.sm_scale,
-                   "tile_config": capi.config_name(cfg)},
+                   "tile_config": tile_config},
         "frac_mfma_peak": round(value / MFMA_PEAK_TFLOPS, 4),
         "latency_ms": {"noncausal_median": round(nc["med"], 5), "noncausal_min": round(nc["mn"], 5),
                        "noncausal_mean": round(nc["mean"], 5),

@@ -29,6 +29,7 @@ EXPORTED = (
     "fl_attn_num_configs",
     "fl_attn_config_name",
     "fl_attn_select_config",
+    "fl_attn_launch_name",
     "fl_attn_fwd_f16_ex",
     "fl_attn_fwd_bf16_ex",
     "fl_attn_splitkv_workspace_bytes",
@@ -106,6 +107,8 @@ def load(path: str = LIB_PATH) -> ctypes.CDLL:
     lib.fl_attn_config_name.restype = ctypes.c_char_p
     lib.fl_attn_select_config.argtypes = [P]
     lib.fl_attn_select_config.restype = ctypes.c_int
+    lib.fl_attn_launch_name.argtypes = [ctypes.POINTER(FlAttnParamsEx), ctypes.c_int32]
+    lib.fl_attn_launch_name.restype = ctypes.c_char_p
     lib.fl_attn_fwd_f16_ex.argtypes = [ctypes.POINTER(FlAttnParamsEx), ctypes.c_int32,
                                        ctypes.c_void_p]
     lib.fl_attn_fwd_f16_ex.restype = ctypes.c_int
@@ -246,6 +249,13 @@ def config_id(name: str) -> int:
 
 def select_config(params: FlAttnParams) -> int:
     return load().fl_attn_select_config(ctypes.byref(params))
+
+
+def launch_name(params: FlAttnParamsEx, dtype: int) -> str | None:
+    """``fl_attn_launch_name``: the kernel the dispatcher launches for `params`
+    in one pass (None if rejected, "" if there is nothing to launch)."""
+    n = load().fl_attn_launch_name(ctypes.byref(params), dtype)
+    return None if n is None else n.decode()
 
 
 def tensor_params(q, k, v, o, sm_scale=0.0, causal=False) -> FlAttnParams:

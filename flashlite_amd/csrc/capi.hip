@@ -649,6 +649,18 @@ int fl_attn_select_config(const fl_attn_params* p) {
   return select_fa2(a);
 }
 
+const char* fl_attn_launch_name(const fl_attn_params_ex* p, int32_t dtype) {
+  const char* who = "fl_attn_launch_name";
+  fl::FwdArgs a;
+  if (dtype != FL_DTYPE_F16 && dtype != FL_DTYPE_BF16)
+    return fail(FL_ERR_INVALID_ARGUMENT, "%s: unknown dtype %d", who, (int)dtype), nullptr;
+  if (check_ex(p, &a, who, /*wide=*/true) != FL_OK) return nullptr;
+  if (empty_problem(a)) return "";
+  a.dtype = dtype == FL_DTYPE_BF16 ? fl::kDtypeBF16 : fl::kDtypeF16;
+  const int c = select_any(a);
+  return c == fl::kRows32Config ? "br32_rows" : fl::kFa2Configs[c].name;
+}
+
 int fl_attn_fwd_f16_cfg(const fl_attn_params* p, int32_t config, void* stream) {
   fl::FwdArgs a;
   int rc = check_fa2(p, &a);

@@ -158,10 +158,9 @@ def main(argv=None):
     if wide:
         p = capi.tensor_params_ex(q, k, v, o, w.sm_scale, bool(args.causal))
         fwd_ex = capi.fwd_bf16_ex if args.dtype == "bf16" else capi.fwd_ex
-        cfg = args.config
     else:
         p = capi.tensor_params(q, k, v, o, w.sm_scale, bool(args.causal))
-        cfg = capi.select_config(p) if args.config < 0 else args.config
+    cfg = args.config
 
     def launch():
         if wide:
@@ -173,7 +172,13 @@ def main(argv=None):
     us = _time_launches(launch, args, torch)
     flops = (2.0 if args.causal else 4.0) * w.batch * w.heads * w.seq ** 2 * head_dim
     nbytes = 4 * w.batch * w.heads * w.seq * head_dim * q.element_size()
-    name = "naive" if args.naive else ("auto" if cfg < 0 else capi.config_name(cfg))
+    if args.naive:
+        name = "naive"
+    elif cfg >= 0:
+        name = capi.config_name(cfg)
+    else:
+        name = capi.launch_name(capi.tensor_params_ex(q, k, v, o, w.sm_scale, bool(args.causal)),
+                                capi.DTYPE_BF16 if args.dtype == "bf16" else capi.DTYPE_F16)
     print(f"{w.name} {args.dtype} D={head_dim} causal={args.causal} {name}"
           f"{' cold' if args.cold_mib else ''}: {us:.2f} us/launch, "
           f"{flops / us / 1e6:.1f} TFLOP/s, {nbytes / us / 1e3:.1f} GB/s", flush=True)

@@ -228,10 +228,15 @@ const char* fl_attn_config_name(int32_t config);
  * configuration should look its id up by name. */
 int fl_attn_config_id(const char* name);
 /* Returns the public table's choice for `p`, or -1 if `p` is rejected (the
- * reason is in fl_attn_last_error()).  fl_attn_fwd_f16 launches it unless a
- * newer measurement favours another one for the shape, which may be internal
- * to the library (32-row groups, for problems of few query rows). */
+ * reason is in fl_attn_last_error()).  This is the table's rule, whose answers
+ * are kept; what a call launches is fl_attn_launch_name's answer. */
 int fl_attn_select_config(const fl_attn_params* p);
+/* The name of the kernel that the dispatcher launches for `p` in one pass
+ * (fl_attn_fwd_f16 and the *_ex entry points with config -1; dtype FL_DTYPE_*):
+ * a configuration's name, or "br32_rows", the 32-row groups, which are
+ * internal to the library and cannot be forced.  NULL if `p` is rejected; ""
+ * if there is no row to compute and nothing is launched. */
+const char* fl_attn_launch_name(const fl_attn_params_ex* p, int32_t dtype);
 
 #ifdef __cplusplus
 }
