@@ -379,27 +379,56 @@ bool config_built(const fl::FwdArgs& a, int cfg) {
   return a.head_dim == 64 && cfg != fl::kCfgW1 && cfg != fl::kCfgW2;
 }
 
-// Head dim 128 (fp16 and bf16 alike; a sweep of 1-128 heads by N 512-8192
-// in bf16, both masks, us per call).  The key-range splits double or
-// quadruple the waves of a problem and halve its longest walk, so they win
-// while they fit one round of the CUs; the groups without a split read each
-// tile for more rows, which counts once the chip is full:
+// Whether a head's work-groups find its K and V in their XCD's L2: wg_coords
+// keeps a head on one XCD only where the work-groups divide evenly over the
+// XCDs, and deals them round-robin otherwise.  That costs nothing while up to
+// 16 heads give every XCD several groups of each, or the chip is half empty;
+// past that the key-range splits and the 32-row groups, which read each tile
+// for fewer rows, fall behind (28 heads of 276 rows over 5678 keys, head dim
+// 64: 252 groups of 32 rows 46.2 us, 140 of 64 rows 33.7; 50 heads of 338 rows
+// over 3640 keys, head dim 128: 300 groups of 64 rows 91.0, 150 of 128 rows 44.8).
+bool l2_local(const fl::FwdArgs& a, int64_t groups) {
+  return groups % fl::device_xcds() == 0 || a.batch_heads <= 16 ||
+         2 * groups <= fl::device_cus();
+}
+
+// The launch rules below choose by numbers of work-groups against the CUs.
+// They were fitted to 5300 shapes at head dim 128 and 13900 at head dim 64
+// (1-256 heads, N 64-16384, N_q 33-N_k, both masks and types, new inputs each
+// call, every configuration timed); figures are us per call.  Square causal
+// problems take one and a half rounds of a split where every XCD carries
+// whole heads (`whole`), so that the heavy blocks go first (wg_coords);
+// otherwise, and where N_q < N_k (nearly equal lengths), a second round is a
+// second round (B4 H32 146 x 3671 causal: 384 groups of 64 rows 47.0, 256 of
+// 128 rows 30.5).
+
+// Head dim 128 (fp16 and bf16 alike).  The key-range splits double or quadruple
+// the waves of a problem and halve its longest walk, so they win while they
+// fit one round of the CUs; the groups without a split read each tile for
+// more rows, which counts once the chip is full:
 //  - at most one 32-row block per CU: the 32-row groups (fa2_rows32.hip; with
-//    384 blocks B2 H12 N512 9.8 against 8.9 for the 64-row split);
-//  - at most one 64-row group per CU, causal 1.5 (their lengths differ):
-//    the split on 64-row groups (B2 H8 N1024 14.3 against 17.4 for the 4-wave
-//    groups, B1 H4 N4096 causal 32.9 against 51.6, B2 H8 N1536 causal 20.5
-//    against 24.0; with 512 groups B2 H8 N2048 42.0 against 35.9);
+//    384 blocks B2 H12 N512 9.8 against 8.9 for the 64-row split), up to 640
+//    keys wherever their K and V come from (18 heads N330 causal, 198 groups, 7.1
+//    against 9.6 for the 128-row groups; 28 heads 193 x 5712, 196 groups, 83.9
+//    against 56.3 for the 64-row split);
+//  - at most one 64-row group per CU, `whole` from 512 keys 1.5: the split on
+//    64-row groups (B2 H8 N1024 14.3 against 17.4 for the 128-row groups, B3 H8
+//    N481 9.3 against 11.1, B1 H4 N4096 causal 32.9 against 51.6, B2 H8 N1536
+//    causal 20.5 against 24.0; with 512 groups B2 H8 N2048 42.0 against 35.9,
+//    and 384 of 76 causal keys, B32 H6, 11.5 against 7.0);
 //  - square causal from 1024 keys with at most one pair of 64-row blocks per
 //    CU: the pairs (B2 H8 N2048 26.5 against 31.0 and 29.4 for the 128-row
 //    split, B1 H4 N8192 76.8 against 101.6 and 89.6; below 1024 keys a pair's
-//    second start-up costs more, B4 H16 N512 15.3 against 13.8);
-//  - from 1536 keys, at most one 128-row group per CU, causal 1.5: the split
-//    on 128-row groups (B2 H8 N1536 24.0 against 24.9, B1 H4 N8192 118
-//    against 127, B2 H8 N3000 causal 43.3 against 49.4; at 1024 keys B2 H16
-//    22.0 against 21.6);
-//  - square causal from 4096 keys with at most one pair of 128-row blocks per
-//    CU: the pairs (B2 H8 N4096 68.4 against 72.1 and 70.1);
+//    second start-up costs more, B4 H16 N512 15.3 against 13.8; not `whole`,
+//    from 2800 keys: B3 H4 N2591 44.0 against 34.7 for the 128-row split);
+//  - from 1100 keys, at most one 128-row group per CU, `whole` 1.5: the split on
+//    128-row groups (B1 H4 N8192 118 against 127, B2 H8 N3000 causal 43.3
+//    against 49.4; below 1536 keys up to 3/4 of a group per CU, B1 H16 N1143
+//    19.2 against 21.2, B2 H16 N1024 22.0 against 21.6);
+//  - square causal from 4096 keys (2000 where not `whole`) with at most one pair
+//    of 128-row blocks per CU: the pairs (B2 H8 N4096 68.4 against 72.1 and 70.1;
+//    B2 H6 N3967 58.1 against 71.3 for the 128-row groups and 82.2 for their
+//    split; 30 heads N2053, 270 pairs, 76.5 against 57.7 for the 128-row groups);
 //  - 256-row groups, non-causal: when one round of them holds what 128-row
 //    groups need a second for (B2 H8 N3000 73.6 against 76.0, B2 H16 N2048
 //    61.2 against 63.9, B2 H16 N3000, two rounds, 149 against 133), and from
@@ -411,90 +440,114 @@ int select_d128(const fl::FwdArgs& a) {
   const int64_t cus = fl::device_cus();
   auto wgs = [&](int64_t br) { return (a.seq + br - 1) / br * (int64_t)a.batch_heads; };
   const bool square = a.causal && a.seq == a.seq_k;
+  const bool whole = a.batch_heads % fl::device_xcds() == 0;
   const int64_t pairs64 = (((int64_t)a.seq + 63) / 64 + 1) / 2 * a.batch_heads;
-  const int64_t most = a.causal ? cus + cus / 2 : cus;
-  if (wgs(32) <= cus && !(a.seq <= 32 && a.batch_heads >= cus)) return fl::kRows32Config;
-  if (wgs(64) <= most) return fl::kCfgSplit2W2;
-  if (square && a.seq_k >= 1024 && pairs64 <= cus) return fl::kCfgPairW2;
-  if (a.seq_k >= 1536 && wgs(128) <= most) return fl::kCfgSplit2;
-  if (square && a.seq_k >= 4096 && wgs(128) <= 2 * cus) return fl::kCfgPair;
+  const int64_t most = square && whole ? cus + cus / 2 : cus;
+  if (wgs(32) <= cus && !(a.seq <= 32 && a.batch_heads >= cus) &&
+      (a.seq_k <= 640 || l2_local(a, wgs(32))))
+    return fl::kRows32Config;
+  if (wgs(64) <= (a.seq_k >= 512 ? most : cus) &&
+      (l2_local(a, wgs(64)) || (square && a.seq_k <= 1024)))
+    return fl::kCfgSplit2W2;
+  if (square && a.seq_k >= (whole ? 1024 : 2800) && pairs64 <= cus) return fl::kCfgPairW2;
+  if (a.seq_k >= 1100 && wgs(128) <= (a.seq_k >= 1536 ? most : 3 * cus / 4)) return fl::kCfgSplit2;
+  const int64_t pairs128 = (((int64_t)a.seq + 127) / 128 + 1) / 2 * a.batch_heads;
+  if (square && a.seq_k >= (whole ? 4096 : 2000) && pairs128 <= cus) return fl::kCfgPair;
   if (!a.causal && wgs(128) > cus && wgs(256) <= cus) return fl::kSlotW8Config;
   if (a.seq_k >= 4096 && wgs(256) >= (a.causal ? 2 : 1) * cus) return fl::kSlotW8Config;
   return fl::kSlotW4Config;
 }
 
-// The base rule of select_d64: fp16 follows the public rule; bf16 does where
-// that picks the streaming kernel, the key quarters, a key-range split or
-// block pairs, and otherwise takes a slot-scheduled group (4 waves for at most
-// 32 query rows over as many heads as CUs: 0-5% faster than 8).
-int select_base(const fl::FwdArgs& a) {
-  const int c = select_fa2(a);
-  if (a.dtype == fl::kDtypeF16 || c == fl::kCfgSplit2 || c == fl::kCfgSplit2W2 ||
-      c == fl::kCfgPair || c == fl::kCfgPairW2 || c == fl::kStreamConfig ||
-      c == fl::kQuarterConfig)
-    return c;
-  const int64_t cus = fl::device_cus();
-  if (a.seq <= 32 && a.batch_heads >= cus) return fl::kSlotW4Config;
-  const int64_t wgs256 = (a.seq + 255) / 256 * (int64_t)a.batch_heads;
-  return (!a.causal && a.seq_k >= 4096 && wgs256 >= cus) ? fl::kSlotW8Config
-                                                           : fl::kSlotW4Config;
-}
-
-// Head dim 64, fp16 and bf16 (sweeps of 1-1024 heads by N 40-8192, both
-// masks, us per call; fp16 figures, bf16 within 3% of them):
-//  - at most one 32-row block per CU, square causal 1.5 (their lengths
-//    differ; 1.25-1.5 non-causal lose 3-11%): the 32-row groups (figures in
-//    fa2_rows32.hip; B2 H8 N640 causal 7.35 against 7.9);
-//  - 257-512 keys with at most two blocks per CU: the key quarters, whose
-//    waves hold both their tiles at once, up to 5/8 of a block per CU (B1 H8
-//    N384 5.05 against 5.35, B1 H16 N300 5.28 against 5.56) and for at most 32
-//    query rows per head up to one (B16 H16 30 x 300 6.9 against 7.8); else
-//    the 32-row groups, two per CU (new inputs each call: B2 H8 N512 6.25
-//    against 7.1, B2 H16 N512 8.2 against 10.8, B30 H10 one row over 400 keys
-//    10.6 against 15.4).  The 64-row split was faster still (B2 H16 N512 7.1
-//    in graphs against 7.8), but only its ranges' first 32 keys set the
-//    stabiliser: 7% more error against 64 bits, 2.88e-4 against 2.70e-4 for
-//    the quarters and 2.66e-4 for the 32-row groups;
-//  - up to 256 keys beyond that: the streaming groups.  The 64-row split (B4
-//    H16 N256 5.95 against 6.3) and the 4-wave groups (B8 H16 N256 7.7 against
-//    9.0) are faster, but sum the p that are rounded to 16 bits;
-//  - at most one 64-row group per CU, causal from 1280 keys 1.5: the 64-row
+// Head dim 64 (fp16 and bf16 alike but for the 256-row groups).  Up to 512
+// keys every choice sums the fp32 p, as the kernels that these calls have
+// always had there do; the slot schedules, which sum the p rounded to 16 bits,
+// are faster in places (B4 H16 N256 5.95 for the 64-row split, B8 H16 N256 7.7
+// against 9.0 for the 4-wave groups, B2 H16 N512 7.5 against 8.4) and up to 7%
+// further from 64 bits.
+//  - up to 256 keys: the streaming groups, but for the 32-row groups past 64
+//    keys (two tiles to share) with at most one block per CU (B2 H12 N172 causal
+//    4.8 against 6.9; 64 keys 4.4 against 4.25; B3 H32 N120 causal, 384 blocks,
+//    6.2 against 5.6), and past 128 keys with two (B2 H32 N234 causal 6.4 against
+//    7.3; not for blocks mostly past the last row, B8 H32 62 x 211 8.6 against
+//    8.3);
+//  - 257-512 keys with at most two 32-row blocks per CU: the key quarters,
+//    whose waves hold both their tiles at once (B1 H8 N384 5.05 against 5.35 for
+//    the 32-row groups, 18 heads N299 causal 5.3 against 6.3, B8 H32 44 x 309
+//    causal 7% faster); the 32-row groups, two per CU, where every XCD carries
+//    whole heads: non-causal or N_q < N_k past 320 keys from one block per CU
+//    (B2 H8 N512 6.25 against 7.1, B1 H32 N510 8.45 against 11.1) and past 448
+//    from 5/8 (5-10%), square causal past 352 keys with more than one (B2 H16
+//    N374 7.1 against 7.6, N512 10%; N337 7.8 against 7.4); at most 32 query rows
+//    per head over more heads than CUs are half of a quarters' group (300 heads of
+//    one row over 400 keys 10.6 against 15.4);
+//  - at most 32 query rows over as many heads as CUs: the 4-wave groups;
+//  - at most one 32-row block per CU, `whole` 1.5: the 32-row groups (figures
+//    in fa2_rows32.hip; B2 H8 N640 causal 7.35 against 7.9), up to 576 keys
+//    also where only they leave few blocks (the pipelined kernels' range, whose
+//    fp32 sums they keep);
+//  - at most one 64-row group per CU, `whole` from 1280 keys 1.5: the 64-row
 //    split (B2 H8 N1280 causal 12.1 against 14.2, B1 H8 N3000 causal 20.1 against
-//    22.0; at N640-768 causal with 1.25-1.5 it lost 10-15%);
-//  - square causal from 1792 keys with at most one pair of 64-row blocks per
-//    CU: the 64-row pairs (B2 H8 N1999 17.9 against 18.4 for the 128-row split;
-//    N1024 over 32 heads 14.3 against 13.4);
-//  - non-causal from 1280 keys with at most one 128-row group per CU: the
-//    128-row split (B2 H8 N1280 12.9 against 14.0; B2 H16 N1024 14.25 against
-//    14.1);
-//  - fp16, non-causal from 2048 keys with more 256-row groups than CUs: those
-//    only from 4096 keys or where their last round is nearly full (B2 H16
-//    N3000, 1.5 rounds, 91.3 against 79.9 on the 4-wave groups).
-// Beyond these, the base rule.
+//    22.0; at N640-768 causal with 1.25-1.5 it lost 10-15%; up to 576 keys only
+//    where the groups divide evenly, B2 H8 N514 8.0 against 8.85 for the 4-wave
+//    groups, 28 heads N515 10.0 against 9.25);
+//  - square causal from 1792 keys (2800 where not `whole`) with at most one pair
+//    of 64-row blocks per CU: the 64-row pairs (B2 H8 N1999 17.9 against 18.4
+//    for the 128-row split, B1 H6 N3961 26.8 against 30.0, 14 heads N2225 21.5
+//    against 20.2; N1024 over 32 heads 14.3 against 13.4);
+//  - from 1280 keys with at most one 128-row group per CU: the 128-row split
+//    (B2 H8 N1280 12.9 against 14.0; B2 H16 N1024 14.25 against 14.1; B32 H8 76 x
+//    1469, one block per head, 21.9 against 19.1, so those from 2048);
+//  - causal beyond: square over 2048-4095 keys up to one and a half rounds the
+//    128-row split, and up to one pair of 128-row blocks per CU the pairs, from
+//    2560 keys square and 4096 otherwise (figures at select_fa2);
+//  - non-causal beyond: 256-row groups, fp16 from 2048 keys with more of them
+//    than half the CUs, below 4096 keys not where their last round is far from
+//    full (B2 H16 N3000, 1.5 rounds, 91.3 against 79.9 on the 4-wave groups), bf16
+//    from 4096 keys with a full round;
+//  - else 128-row groups of 4 waves, two per CU.
 int select_d64(const fl::FwdArgs& a) {
   const int64_t cus = fl::device_cus();
   auto wgs = [&](int64_t br) { return (a.seq + br - 1) / br * (int64_t)a.batch_heads; };
   const bool square = a.causal && a.seq == a.seq_k;
+  const bool whole = a.batch_heads % fl::device_xcds() == 0;
   const bool few = a.seq <= 32 && a.batch_heads >= cus;  // decode over many heads
-  const bool quarter =
-      !fl::stream_config_fits(a) && fl::quarter_config_fits(a) && wgs(32) <= 2 * cus;
-  if (quarter) {
-    const bool keep = 8 * wgs(32) <= 5 * cus || (a.seq <= 32 && wgs(32) <= cus);
-    return keep ? fl::kQuarterConfig : fl::kRows32Config;
+  const int64_t blocks = wgs(32);
+  if (fl::stream_config_fits(a)) {
+    const bool rows32 = blocks <= cus ? a.seq_k > 64 && !few
+                                      : a.seq_k > 128 && blocks <= 2 * cus && a.seq > 96;
+    return rows32 ? fl::kRows32Config : fl::kStreamConfig;
   }
-  if (!few && wgs(32) <= (square ? cus + cus / 2 : cus)) return fl::kRows32Config;
-  if (fl::stream_config_fits(a)) return fl::kStreamConfig;
+  if (fl::quarter_config_fits(a) && blocks <= 2 * cus) {
+    bool rows32 = false;
+    if (a.seq <= 32)
+      rows32 = blocks > cus;
+    else if (whole && a.seq > 48)
+      rows32 = square ? a.seq_k > 352 && blocks > cus
+                      : (a.seq_k > 320 && blocks >= cus) ||
+                            (a.seq_k > 448 && 8 * blocks >= 5 * cus);
+    return rows32 ? fl::kRows32Config : fl::kQuarterConfig;
+  }
   if (few) return fl::kSlotW4Config;
-  if (wgs(64) <= (a.causal && a.seq_k >= 1280 ? cus + cus / 2 : cus)) return fl::kCfgSplit2W2;
+  const int64_t most = square && whole ? cus + cus / 2 : cus;
+  if (blocks <= most && (l2_local(a, blocks) || (a.seq_k <= 576 && 4 * wgs(128) < cus)))
+    return fl::kRows32Config;
+  if (wgs(64) <= (a.seq_k >= 1280 ? most : cus) &&
+      (a.seq_k > 576 || wgs(64) % fl::device_xcds() == 0))
+    return fl::kCfgSplit2W2;
   const int64_t pairs64 = (((int64_t)a.seq + 63) / 64 + 1) / 2 * a.batch_heads;
-  if (square && a.seq_k >= 1792 && pairs64 <= cus) return fl::kCfgPairW2;
-  if (!a.causal && a.seq_k >= 1280 && wgs(128) <= cus) return fl::kCfgSplit2;
-  const int c = select_base(a);
-  const int64_t g = wgs(256), rounds = (g + cus - 1) / cus;
-  if (a.dtype == fl::kDtypeF16 && c == fl::kSlotW8Config && a.seq_k < 4096 && rounds > 1 &&
-      10 * g < 9 * rounds * cus)
+  if (square && a.seq_k >= (whole ? 1792 : 2800) && pairs64 <= cus) return fl::kCfgPairW2;
+  if (wgs(128) <= cus && a.seq_k >= (a.seq > 128 ? 1280 : 2048)) return fl::kCfgSplit2;
+  if (a.causal) {
+    if (square && a.seq_k >= 2048 && a.seq_k < 4096 && wgs(128) <= cus + cus / 2)
+      return fl::kCfgSplit2;
+    if (a.seq_k >= (square ? 2560 : 4096) && wgs(128) <= 2 * cus) return fl::kCfgPair;
     return fl::kSlotW4Config;
-  return c;
+  }
+  const int64_t g = wgs(256), rounds = (g + cus - 1) / cus;
+  if (a.dtype == fl::kDtypeBF16)
+    return a.seq_k >= 4096 && g >= cus ? fl::kSlotW8Config : fl::kSlotW4Config;
+  const bool ragged = a.seq_k < 4096 && rounds > 1 && 10 * g < 9 * rounds * cus;
+  return a.seq_k >= 2048 && 2 * g > cus && !ragged ? fl::kSlotW8Config : fl::kSlotW4Config;
 }
 
 int select_any(const fl::FwdArgs& a) {

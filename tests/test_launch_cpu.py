@@ -48,3 +48,51 @@ def test_lse_does_not_change_the_kernel(dtype):
                 for causal in (False, True):
                     args = (heads, nq, nk, d, causal)
                     assert launched(*args, dtype=dtype) == launched(*args, lse=8 * A, dtype=dtype)
+
+
+# (heads, N_q, N_k, head dim, causal) -> the kernel that measured fastest among
+# those that lose no precision there; the figures are beside the rules.
+CHOICES = [
+    # head dim 64, up to 256 keys
+    (30, 64, 64, 64, True, STREAM), (24, 172, 172, 64, True, ROWS32),
+    (96, 120, 120, 64, True, STREAM), (64, 234, 234, 64, True, ROWS32),
+    (256, 62, 211, 64, False, STREAM), (128, 256, 256, 64, False, STREAM),
+    # 257-512 keys
+    (18, 299, 299, 64, True, QUARTER), (8, 384, 384, 64, False, QUARTER),
+    (25, 300, 300, 64, False, QUARTER), (256, 44, 309, 64, True, QUARTER),
+    (32, 337, 337, 64, True, QUARTER), (32, 374, 374, 64, True, ROWS32),
+    (32, 510, 510, 64, False, ROWS32), (300, 1, 400, 64, False, ROWS32),
+    (64, 512, 512, 64, False, W4),
+    # longer ranges
+    (28, 276, 5678, 64, True, SPLIT64), (10, 772, 12304, 64, True, ROWS32),
+    (128, 146, 3671, 64, True, SPLIT128), (10, 2107, 2107, 64, True, SPLIT128),
+    (8, 3000, 3000, 64, True, SPLIT64), (16, 1999, 1999, 64, True, PAIR64),
+    (14, 2225, 2225, 64, True, SPLIT128), (6, 3961, 3961, 64, True, PAIR64),
+    (28, 515, 515, 64, False, W4), (16, 514, 514, 64, False, SPLIT64),
+    (256, 76, 1469, 64, False, W4), (32, 3000, 3000, 64, False, W4),
+    # head dim 128
+    (18, 330, 330, 128, True, ROWS32), (28, 193, 5712, 128, False, SPLIT64),
+    (192, 76, 76, 128, True, W4), (50, 338, 3640, 128, True, SPLIT128),
+    (16, 1536, 1536, 128, True, SPLIT64), (12, 2591, 2591, 128, True, SPLIT128),
+    (12, 3967, 3967, 128, True, PAIR128), (30, 2053, 2053, 128, True, W4),
+    (16, 3000, 3000, 128, True, SPLIT128), (16, 8192, 8192, 128, False, W8),
+]
+
+
+@pytest.mark.parametrize("heads,nq,nk,d,causal,name", CHOICES)
+def test_choices(heads, nq, nk, d, causal, name):
+    assert launched(heads, nq, nk, d, causal) == name
+
+
+def test_short_key_ranges_sum_unrounded_p():
+    """Up to 512 keys (head dim 64) with at most two 32-row blocks per CU, and
+    up to 256 for any count, only kernels whose row sums take the fp32 p."""
+    for heads in (1, 7, 16, 25, 64, 100, 255, 256, 300, 511, 512, 1024):
+        for nq in (1, 5, 32, 33, 64, 96, 100, 200, 256, 400, 512):
+            for nk in (1, 64, 65, 128, 129, 193, 256, 257, 320, 352, 448, 512):
+                if nk > 256 and heads * -(-nq // 32) > 512:
+                    continue
+                for causal in (False, True):
+                    for dtype in (capi.DTYPE_F16, capi.DTYPE_BF16):
+                        assert launched(heads, nq, nk, 64, causal, dtype=dtype) in (
+                            ROWS32, STREAM, QUARTER)
