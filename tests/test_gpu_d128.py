@@ -37,7 +37,7 @@ def run_shared_kv(kind, h, nq, nk, d, causal, dev, seed, sm=0.1, qk_scale=1.0, b
     fn = capi.fwd_bf16_ex if kind == "bf16" else capi.fwd_ex
     capi.check(fn(p, torch.cuda.current_stream(dev).cuda_stream, -1))
     torch.cuda.synchronize(dev)
-    assert torch.isfinite(o.float()).all() or nq > nk, "unwritten rows"
+    assert torch.isfinite(o.float()).all(), "unwritten rows"
     kk, vv = (np.repeat(x[:, :1], len(checked), axis=1) for x in (k, v))
     rows = sample_rows(nq, count=64, seed=seed) if nq > 1200 else np.arange(nq)
     out = o[:, checked].float().cpu().numpy()
@@ -55,35 +55,60 @@ def run_shared_kv(kind, h, nq, nk, d, causal, dev, seed, sm=0.1, qk_scale=1.0, b
         assert lmean <= LSE_MEAN_ABS[kind]
 
 
-# (heads, N_q, N_k, causal): the configuration the dispatcher takes.
+# What the dispatcher launches (asserted on an MI355X seen whole): shapes as
+# (heads, N_q, N_k, causal).  Ragged and single-row ends, key ranges of one
+# tile (the second stream of a split has none), rows with no visible key.
 SHAPES = {
-    "64-row split": [(3, 1, 1, False), (3, 33, 31, True), (3, 65, 64, True), (4, 130, 1025, False),
-                     (16, 512, 700, True), (50, 450, 450, True), (3, 100, 37, True)],
-    "64-row pairs": [(28, 1025, 1025, True), (26, 1089, 1089, True)],
-    "128-row split": [(70, 200, 1537, False), (100, 250, 1600, True), (70, 257, 1568, False)],
-    "128-row pairs": [(12, 4097, 4097, True)],
-    "256-row groups": [(100, 300, 100, False), (512, 33, 4099, True), (256, 40, 4096, False)],
-    "128-row groups": [(300, 100, 97, False), (300, 130, 65, True), (200, 300, 301, True)],
+    "br32_rows": [(3, 1, 1, False), (3, 33, 31, True), (3, 65, 64, True), (4, 130, 1025, False),
+                  (16, 512, 700, True), (3, 100, 37, True)],
+    "br64_bc64_w2x2_slot": [(40, 300, 301, True), (60, 200, 97, False), (120, 65, 31, True),
+                            (48, 260, 1000, True), (40, 513, 513, True), (64, 200, 130, False),
+                            (256, 40, 4096, False)],
+    "br64_bc64_w2x2_pair": [(24, 1025, 1025, True), (24, 1089, 1089, True),
+                            (10, 2817, 2817, True)],
+    "br128_bc64_w4x2_slot": [(70, 200, 1537, False), (100, 250, 1600, True), (70, 257, 1568, False),
+                             (60, 257, 1101, False)],
+    "br128_bc64_w4x2_pair": [(12, 4097, 4097, True)],
+    "br256_bc64_w8_slot": [(100, 300, 100, False), (512, 33, 4099, True), (300, 40, 4096, False)],
+    "br128_bc64_w4_slot": [(300, 100, 97, False), (300, 130, 65, True), (200, 300, 301, True),
+                           (50, 450, 450, True)],
 }
+CASES = [(name, *s) for name, v in SHAPES.items() for s in v]
+
+
+def assert_launch(name, kind, h, nq, nk, causal, dev):
+    """`name` is what a call of this shape launches, where all CUs are seen."""
+    import torch
+
+    if torch.cuda.get_device_properties(dev).multi_processor_count != 256:
+        return
+    base = capi.make_params(1 << 16, 1 << 17, 1 << 18, 1 << 19, 1, h, nq, nk, 128, 0.1, causal)
+    qs, ks = (h * nq * 128, nq * 128, 128), (h * nk * 128, nk * 128, 128)
+    p = capi.make_params_ex(base, qs, ks, ks, qs)
+    assert capi.launch_name(p, capi.DTYPE_BF16 if kind == "bf16" else capi.DTYPE_F16) == name
 
 
 @pytest.mark.parametrize("kind", ["fp16", "bf16"])
-@pytest.mark.parametrize("h,nq,nk,causal", [s for v in SHAPES.values() for s in v])
-def test_dispatched_shapes(cuda, kind, h, nq, nk, causal):
+@pytest.mark.parametrize("name,h,nq,nk,causal", CASES)
+def test_dispatched_shapes(cuda, kind, name, h, nq, nk, causal):
+    assert_launch(name, kind, h, nq, nk, causal, cuda)
     run_shared_kv(kind, h, nq, nk, 128, causal, cuda, seed=h + 7 * nq + nk)
 
 
 # Scores far above the first tile's best hand the block to the checked pass.
 @pytest.mark.parametrize("kind", ["fp16", "bf16"])
-@pytest.mark.parametrize("h,nq,nk,causal", [SHAPES["64-row split"][3], SHAPES["64-row pairs"][0],
-                                            SHAPES["128-row split"][1],
-                                            SHAPES["128-row groups"][2]])
-def test_peaked(cuda, kind, h, nq, nk, causal):
+@pytest.mark.parametrize("name,i", [("br32_rows", 3), ("br64_bc64_w2x2_slot", 3),
+                                    ("br64_bc64_w2x2_pair", 0), ("br128_bc64_w4x2_slot", 1),
+                                    ("br128_bc64_w4_slot", 2)])
+def test_peaked(cuda, kind, name, i):
+    h, nq, nk, causal = SHAPES[name][i]
+    assert_launch(name, kind, h, nq, nk, causal, cuda)
     run_shared_kv(kind, h, nq, nk, 128, causal, cuda, seed=h + nq, sm=1.0, qk_scale=2.0)
 
 
 def test_projection_layout_and_negative_scale(cuda):
-    run_shared_kv("bf16", 28, 1025, 1025, 128, True, cuda, seed=5, sm=-0.1, bnhd=True)
+    run_shared_kv("bf16", 24, 1025, 1025, 128, True, cuda, seed=5, sm=-0.1, bnhd=True)
+    run_shared_kv("bf16", 40, 300, 301, 128, True, cuda, seed=7, sm=-0.1, bnhd=True)
     run_shared_kv("fp16", 100, 250, 1600, 128, True, cuda, seed=6, sm=-0.1, bnhd=True)
 
 

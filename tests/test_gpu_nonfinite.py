@@ -134,6 +134,6 @@ def test_one_pass(cuda, kind, config, causal):
 # 64-row split, 64-row pairs, 128-row split; and the 128-row groups by id.
 @pytest.mark.parametrize("h,nq,nk,causal,config", [
     (HEADS, 100, 700, True, -1), (40, 300, 301, True, -1), (40, 300, 301, False, -1),
-    (28, 1025, 1025, True, -1), (100, 250, 1600, True, -1), (HEADS, 300, 301, True, SLOT_W4_CFG)])
+    (24, 1025, 1025, True, -1), (100, 250, 1600, True, -1), (HEADS, 300, 301, True, SLOT_W4_CFG)])
 def test_head_dim_128(cuda, h, nq, nk, causal, config):
     run("bf16", 128, h, nq, nk, causal, cuda, one_pass(config))

@@ -1,7 +1,7 @@
 """GPU parity of the 32-row groups (few query blocks: the key tiles dealt to
-4 or 8 waves) at both head dims and element types, through the dispatcher,
-at the edges of tiles, of the waves' shares and of the 8-wave rule (2048
-keys).  Tolerances: gpu_util (against the fp32 oracle).
+4 or 8 waves) at both head dims and element types, through the dispatcher
+(which at head dim 64 takes the streaming groups up to 64 keys), at the edges
+of tiles, of the waves' shares and of the 8-wave rule (2048 keys).  Tolerances: gpu_util (against the fp32 oracle).
 """
 
 import numpy as np
@@ -18,7 +18,8 @@ KINDS = [("fp16", 64), ("fp16", 128), ("bf16", 64), ("bf16", 128)]
 # N_q, N_k: single rows and keys, block edges, fewer tiles than waves, ragged
 # tails, rows with no visible key (N_q > N_k), 8-wave groups.
 SHAPES = [(1, 1), (1, 255), (31, 64), (32, 65), (33, 33), (64, 193), (40, 256), (100, 37),
-          (65, 700), (5, 1000), (33, 2047), (32, 2048), (70, 2113)]
+          (65, 700), (5, 1000), (33, 2047), (32, 2048), (70, 2113),
+          (1, 66), (100, 70), (95, 129)]
 
 
 def check(kind, d, nq, nk, sm, causal, dev, scale=1.0, views=None, h=3):
@@ -102,9 +103,11 @@ def test_one_kernel_with_and_without_lse(cuda, kind, h, nq, nk, causal):
 
 @pytest.mark.parametrize("kind", ["fp16", "bf16"])
 @pytest.mark.parametrize("causal", [False, True])
-@pytest.mark.parametrize("h,nq,nk", [(12, 700, 257), (16, 1024, 512), (264, 20, 300)])
+@pytest.mark.parametrize("h,nq,nk", [(12, 700, 257), (16, 1024, 512), (264, 20, 300),
+                                     (16, 700, 400), (16, 700, 200)])
 def test_two_groups_per_cu(cuda, kind, causal, h, nq, nk):
-    """257-512 keys over one to two 32-row blocks per CU: two tiles per wave,
-    the second of which raises the stabiliser in about half the rows."""
+    """129-512 keys over one to two 32-row blocks per CU (12 heads of 700 x 257:
+    the key quarters): up to two tiles per wave, the second of which raises the
+    stabiliser in about half the rows."""
     check(kind, 64, nq, nk, 0.125, causal, cuda, h=h)
     check(kind, 64, nq, nk, 1.0, causal, cuda, scale=1.5, h=h)

@@ -30,6 +30,16 @@ def test_wide_plan(dtype, d):
                 assert n * heads <= 512 and 4 * n <= tiles or n == 0 or n == 8
 
 
+@pytest.mark.parametrize("dtype,d,heads,nq,nk,chunks", [
+    (capi.DTYPE_F16, 128, 16, 1, 4096, 8), (capi.DTYPE_BF16, 64, 16, 1, 4096, 8),
+    (capi.DTYPE_BF16, 128, 64, 1, 3000, 4), (capi.DTYPE_BF16, 64, 64, 1, 4096, 4),
+    (capi.DTYPE_BF16, 64, 64, 1, 3000, 0), (capi.DTYPE_F16, 128, 2, 32, 16384, 32),
+    (capi.DTYPE_BF16, 128, 1, 7, 100000, 195), (capi.DTYPE_F16, 128, 127, 1, 4096, 4)])
+def test_wide_chunk_counts(dtype, d, heads, nq, nk, chunks):
+    row = 4 * (68 if d == 64 else 132)
+    assert need(dtype, d, heads, nq, nk) == chunks * heads * nq * row
+
+
 def test_fp16_d64_follows_the_split_plan():
     for heads, nq, nk in [(16, 1, 4096), (16, 4, 8192), (1024, 1, 4096), (16, 4096, 4096), (8, 64, 8192)]:
         base = capi.make_params(0x10000, 0x20000, 0x30000, 0x40000, 1, heads, nq, nk, 64, 0.1, False)
