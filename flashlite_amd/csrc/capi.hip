@@ -106,8 +106,8 @@ int check_pointers(const fl_attn_params* p, fl::FwdArgs* a, const char* who, uin
 }
 
 // The public table's rule: what fl_attn_select_config reports (its answers for
-// given shapes are part of the interface), and the base of select_d64, which
-// launches by newer measurements where they differ.
+// given shapes are part of the interface).  Launches follow select_d64 and
+// select_d128, newer measurements of more kernels.
 //
 // Tile-configuration choice for the device's CUs (fl::device_cus(): 256 on
 // an MI355X seen whole, where the rules below were measured; every
@@ -368,8 +368,9 @@ hipError_t run_kvsplit(const fl::FwdArgs& a, const KvPlan& plan, float* part, hi
                       : fl::launch_kvsplit(a, plan.waves, part, plan.nsplit, st);
 }
 
-// fp16 at head_dim 64 has every tile configuration; bf16 at head_dim 64
-// all but the two pipelined ones; head_dim 128 the two slot-scheduled ones.
+// What a caller can force: fp16 at head_dim 64 every tile configuration; bf16
+// at head_dim 64 all but the two pipelined ones; head_dim 128 the two
+// slot-scheduled ones (its splits and pairs are launched by rule only).
 bool narrow_configs(const fl::FwdArgs& a) {
   return a.dtype != fl::kDtypeF16 || a.head_dim != 64;
 }
@@ -458,10 +459,10 @@ int select_d128(const fl::FwdArgs& a) {
   return fl::kSlotW4Config;
 }
 
-// Head dim 64 (fp16 and bf16 alike but for the 256-row groups).  Up to 512
-// keys every choice sums the fp32 p, as the kernels that these calls have
-// always had there do; the slot schedules, which sum the p rounded to 16 bits,
-// are faster in places (B4 H16 N256 5.95 for the 64-row split, B8 H16 N256 7.7
+// Head dim 64 (fp16 and bf16 alike but for the 256-row groups).  Up to 256
+// keys, and for 257-512 with at most two 32-row blocks per CU, every choice sums
+// the fp32 p, as the public table's do there; the slot schedules, which sum
+// the p rounded to 16 bits, are faster in places (B4 H16 N256 5.95 for the 64-row split, B8 H16 N256 7.7
 // against 9.0 for the 4-wave groups, B2 H16 N512 7.5 against 8.4) and up to 7%
 // further from 64 bits.
 //  - up to 256 keys: the streaming groups, but for the 32-row groups past 64

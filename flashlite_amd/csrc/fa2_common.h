@@ -49,8 +49,8 @@
 // exact math since softmax is shift invariant; m never exceeds the running
 // max, so the row sum stays >= 1).  p is packed to fp16 for GEMM2.  Row
 // sums: the reference sums the unrounded fp32 p (kernel_flash2.cu:268-276,
-// :339), as the pipelined, streaming, key-quarter and head_dim-128 kernels
-// here do (each lane sums its own keys and the two halves of a row meet
+// :339), as the pipelined, streaming, key-quarter, 32-row and head_dim-128
+// kernels here do (each lane sums its own keys and the two halves of a row meet
 // once, in the epilogue); the slot schedules sum the rounded p that GEMM2
 // multiplies, in fp32 on the matrix core (Rows::init_msum).
 //
@@ -69,7 +69,14 @@
 //                   and their combine kernel.
 //   fa2_stream.hip  N_k <= 256: one persistent 8-wave work-group per CU
 //                   walks whole units through two LDS buffers.
-//   fa2_d128.hip    head_dim 128: the slot schedule over 32-key tiles.
+//   fa2_short.hip   N_k <= 512: one 32-row block per work-group, a quarter of
+//                   the keys per wave.
+//   fa2_rows32.hip  one 32-row block per work-group, the key tiles dealt to 4
+//                   or 8 waves, each through slots of its own; both head
+//                   dims, split-KV chunks too.
+//   fa2_d128_kernel.h  head_dim 128 (row state: fa2_d128.h; instances:
+//                   fa2_d128.hip fp16, fa2_d128_bf16.hip): the slot schedule
+//                   over 32-key tiles, its key-range splits and block pairs.
 //
 // Causal.  Keys after a lane's query and keys >= N are masked to -inf on the
 // diagonal and tail tiles only; work-groups are fed to each XCD heaviest
@@ -79,7 +86,8 @@
 // K with (row&7)^((row>>3)&1), V with 2*(row&3), which makes the GEMM1
 // ds_read_b128 pattern, the GEMM2 ds_read_b64_tr_b16 pattern and the
 // row-contiguous tile writes conflict-free (0 SQ_LDS_BANK_CONFLICT measured
-// for the D = 64 kernels).
+// in the D = 64 kernels but for a few cycles per wave in the pairs' and the
+// split-KV quarters' merges).
 
 #pragma once
 

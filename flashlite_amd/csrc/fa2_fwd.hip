@@ -1,7 +1,7 @@
 // Tile configurations of the FA2 forward and their dispatch to the
 // schedule that implements each (fa2_pipe.hip, fa2_slot.hip, fa2_stream.hip,
-// fa2_short.hip, fa2_d128.hip, fa2_rows32.hip).  The dispatcher that picks a configuration for a problem is
-// capi.hip's select_fa2.
+// fa2_short.hip, fa2_rows32.hip, fa2_d128_kernel.h).  The rules that pick one
+// for a problem are capi.hip's select_d64 and select_d128.
 
 #include "fl_internal.h"
 

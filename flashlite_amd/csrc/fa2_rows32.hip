@@ -23,12 +23,12 @@ namespace {
 // eight) independent chains per block shorten it to a quarter (or an eighth)
 // of the tiles, where the 64-row split halves it.  NW = 4 keeps 64 KiB of
 // tiles, two groups per CU; NW = 8, one group per CU, serves long walks.
-// Against the configurations the dispatcher took before (fp16 and bf16 alike
-// at head dim 64, us per call): B1 H1 N128 5.05 -> 4.35, B2 H8 N256 7.2 ->
-// 4.8, B2 H8 N512 7.0 -> 5.8, B1 H8 N1024 8.9 -> 6.9, B1 H2 N4096 causal 21.4
-// -> 14.2 (NW = 8; 15.9 with 4), B1 H1 N8192 36.8 -> 29.4; head dim 128: B2
-// H8 N512 8.55 -> 6.97, B1 H2 N4096 30.9 -> 25.6.  Two tiles in flight per
-// wave (128 KiB, one group per CU) measured 0-10% slower than one.
+// Against the configurations launched before it (fp16, us per call in a graph,
+// new inputs each call): B1 H1 N128 4.66 -> 4.04, B2 H8 N256 6.8 -> 4.6, B2 H8
+// N512 7.1 -> 5.9, B1 H8 N1024 9.2 -> 7.5 (bf16 9.4 -> 7.6), B1 H2 N4096 causal
+// 22.9 -> 16.2, B1 H1 N8192 44.3 -> 31.9; head dim 128: B2 H8 N512 12.6 -> 7.45,
+// B1 H2 N4096 54.3 -> 28.5.  Two tiles in flight per wave (128 KiB, one group
+// per CU) measured 0-10% slower than one.
 template <int D, class T, bool CAUSAL>
 struct TileRows;
 
