@@ -462,9 +462,9 @@ int select_d128(const fl::FwdArgs& a) {
 // Head dim 64 (fp16 and bf16 alike but for the 256-row groups).  Up to 256
 // keys, and for 257-512 with at most two 32-row blocks per CU, every choice sums
 // the fp32 p, as the public table's do there; the slot schedules, which sum
-// the p rounded to 16 bits, are faster in places (B4 H16 N256 5.95 for the 64-row split, B8 H16 N256 7.7
-// against 9.0 for the 4-wave groups, B2 H16 N512 7.5 against 8.4) and up to 7%
-// further from 64 bits.
+// the p rounded to 16 bits, are faster in places (64-row split: B4 H16 N256
+// 5.95 against 6.3, B2 H16 N512 7.5 against 8.4; 4-wave groups: B8 H16 N256 7.7
+// against 9.0) and up to 7% further from 64 bits.
 //  - up to 256 keys: the streaming groups, but for the 32-row groups past 64
 //    keys (two tiles to share) with at most one block per CU (B2 H12 N172 causal
 //    4.8 against 6.9; 64 keys 4.4 against 4.25; B3 H32 N120 causal, 384 blocks,
